@@ -181,7 +181,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                                         RfLds<CAP>& sh) {
     constexpr bool WIN = MODE >= 1;     // meshes beyond the vertex cache, window by window
     constexpr bool FRAMES = MODE == 2;  // and the frame dump (stage calls)
-    constexpr int SPT = 2048 / BT;  // fitness slots per thread
+    constexpr int PR = 1024 / BT;  // pairs of fitness slots per thread
     int32_t* const lds = sh.lds;
     int32_t* const s_box = sh.s_box;
     int32_t* const s_stale = sh.s_stale;
@@ -469,9 +469,9 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     const int32_t MW = full ? 0 : (TW + 31) >> 5;  // mask words per tile row
     const bool col_line = minX >= tx0 && minX < tx1;
 
-    float acc_e[SPT];
+    float acc_e[PR][2];  // [i][j]: slot 2 (tid + i BT) + j
 #pragma unroll
-    for (int j = 0; j < SPT; ++j) acc_e[j] = 0.0f;
+    for (int i = 0; i < PR; ++i) acc_e[i][0] = acc_e[i][1] = 0.0f;
     uint32_t n_seg = 0, n_tr = 0, n_rend = 0;
     unsigned long long px_r = 0;
 
@@ -1031,111 +1031,141 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         const int32_t qx0 = max(dx0, rx0), qx1 = min(dx1, rx1);
         const int32_t qy0 = max(db0, ry0), qy1 = min(db1, ry1);
         if (DW > 0 && qx0 < qx1 && qy0 < qy1) {
-            const int32_t k0 = qy0 - minY, k1 = qy1 - minY;
-            const int32_t tlo = min(k0 * W + (qx0 - minX), T);
-            const int32_t thi = min(k1 * W + 1, T);
-            // U steps of 2048 per batch: all their loads go out before the
-            // first sum (a pixel outside Q reads as empty and observed 0,
-            // which adds nothing), then each slot sums in increasing t
-            constexpr int U = SPT >= 8 ? 1 : 8 / SPT;
-            // Q in union-box offsets (x, y), and the tile and crop indices as
-            // y * pitch + x + constant
-            const int32_t qxa = qx0 - minX, qxb = qx1 - minX, qya = qy0 - minY, qyb = qy1 - minY;
-            // (minY - db0 can reach -2^23 - 480, beyond __mul24: wrapping 32-bit
-            // products, exact modulo 2^32, as is each index they add up to)
-            const int32_t tc = (minY - db0) * DW + (minX - dx0), oc = (minY - ry0) * rw + (minX - rx0);
-            // Thread tid walks t = t0 + m BT (m = 0, 1, ...; slot j = m mod SPT)
-            // and keeps the true quotient and remainder y, x of t by W from
-            // step to step (BT = sq W + sr).  The fp32 row index differs from
-            // the true one only at t = yW (x = 0): for t below 2^23 the
-            // product t rcp(W) carries a relative error under 2^-23, less
-            // than x / t for 0 < x < W.  There it is y - 1 when row y is
-            // "short", and t visits (0, y - 1); column 0 of the union box lies
-            // in Q only when qxa = 0.  A t inside Q in (x, y) is at least tlo
-            // and below k1 W + 1, so of [tlo, thi) only t < T is left to test,
-            // and only in the last batch: every t of an earlier one is below
-            // its end, at most thi.  The four forms (column 0 in Q or not,
-            // last batch or not) are compiled apart.
-            const uint32_t xn = (uint32_t)(qxb - qxa), yn = (uint32_t)(qyb - qya);
-            const int32_t sq = BT / W, sr = BT - sq * W;
+            // Thread tid takes the slot pairs 2 (tid + i BT), i < PR: its t are
+            // consecutive pixels of a row (t, t + 1), so a pair shares its
+            // addressing, its range test and its loads (two words of the
+            // tile, one unaligned word of the crop).  VALU issue bounds this
+            // scan; with addressing of its own a pixel took 31 instructions,
+            // now 13 (one solve of 256 particles, 220x220 rect, 100
+            // iterations: 8.73 -> 8.19 ms).
+            constexpr int U = PR >= 4 ? 1 : 4 / PR;  // 2048-slot rounds a batch: four pairs in flight
+            constexpr int kStep = 2 * BT;            // t from one pair of a thread to its next
+            // Q in union-box offsets: columns [qxa, qxa + xn), rows [ka, kb),
+            // i.e. t in [ka W, kb W), all below T (kb <= H: a rect row lies
+            // above the box's last)
+            const int32_t qxa = qx0 - minX, ka = qy0 - minY, kb = qy1 - minY;
+            const uint32_t xn = (uint32_t)(qx1 - qx0);
+            const int32_t ta = ka * W;
+            const uint32_t tn = (uint32_t)(kb * W - ta);
+            const int32_t base0 = ((ta + qxa) / 2048) * 2048, thi = kb * W + 1;
+            // The fp32 row index differs from the true one only at t = yW
+            // (x = 0): for t below 2^23 the product t rcp(W) carries a
+            // relative error under 2^-23, less than x / t for 0 < x < W.
+            // There it is y - 1 when row y is "short", and t visits (0, y - 1).
+            // Column 0 of the union box lies in Q only when qxa = 0; a pair
+            // that runs over its row's end then meets it too.  Those pixels
+            // are looked up apart (a wave meets one per W values of t).  Only
+            // a batch that reaches outside [ka W, kb W) tests rows.  The four
+            // forms (column 0 in Q or not, such a batch or not) are compiled
+            // apart.
             const bool col0 = qxa == 0;
-            // the crop addressed by a 32-bit byte offset from its base
-            const QG char* __restrict__ ob = (const QG char*)obs;
-            int32_t y, x;
+            const int32_t sq = kStep / W, sr = kStep - sq * W;
+            // x - qxa of the pair's first pixel; its byte offsets in the tile
+            // and, from two bytes before the crop (a pair may start one pixel
+            // left of Q), in the crop.  All step by constants, others over a
+            // row's end (wrapping arithmetic; used only inside Q).
+            int32_t xq, y, to, oo;
             {
-                const int32_t t = (tlo / 2048) * 2048 + tid;
+                const int32_t t = base0 + 2 * tid;
                 y = row_of(t, vis.rW);
-                x = t - y * W;
+                int32_t x = t - y * W;
                 if (x >= W) { x -= W; ++y; }
+                xq = x - qxa;
+                to = 4 * ((y - (db0 - minY)) * DW + x - (dx0 - minX));
+                oo = 2 * ((y - (ry0 - minY)) * rw + x - (rx0 - minX)) + 2;
             }
-            // the three counters per wave, from ballots (scalar adds)
-            uint32_t w_rend = 0, w_tr = 0, w_seg = 0;
-            auto batch = [&](int32_t base, auto c0, auto last) {
-                constexpr bool kCol0 = decltype(c0)::value, kLast = decltype(last)::value;
-                int32_t zr[U][SPT], zk[U][SPT];
+            // wrap-dependent steps, kept in vector registers: a select takes
+            // them without a move
+            int32_t x0s = sr, x1s = sr - W;
+            int32_t to0 = 4 * (sq * DW + sr), to1 = to0 + 4 * (DW - W);
+            int32_t oo0 = 2 * (sq * rw + sr), oo1 = oo0 + 2 * (rw - W);
+            __asm__("" : "+v"(x0s), "+v"(x1s), "+v"(to0), "+v"(to1), "+v"(oo0), "+v"(oo1));
+            const int32_t xlim = W - qxa - sr;
+            typedef uint32_t u32_2 __attribute__((aligned(2)));
+            const QG char* __restrict__ ob = (const QG char*)obs - 2;
+            const char* const tb = reinterpret_cast<const char*>(tile);
+            // rendered, observed and both: counted per wave from ballots
+            uint32_t w_rend = 0, w_obs = 0, w_both = 0;
+            // the pairs in flight: depths, observed depths (two halves; lanes
+            // outside Q keep what they held, masked below), Q's lanes
+            int32_t zr[U * PR][2] = {};
+            uint32_t zk[U * PR] = {};
+            uint64_t in[U * PR][2];
+            auto batch = [&](int32_t base, auto c0, auto edge) {
+                constexpr bool kCol0 = decltype(c0)::value, kEdge = decltype(edge)::value;
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
+                for (int i = 0; i < U * PR; ++i) {
+                    const int32_t t = base + i * kStep + 2 * tid;
+                    in[i][0] = __ballot((uint32_t)xq < xn);
+                    in[i][1] = __ballot((uint32_t)(xq + 1) < xn);
+                    if (kEdge) {
+                        const uint64_t row = __ballot((uint32_t)(t - ta) < tn);
+                        in[i][0] &= row;
+                        in[i][1] &= row;
+                    }
+                    if (__builtin_amdgcn_inverse_ballot_w64(in[i][0] | in[i][1])) {
+                        const int32_t* z = reinterpret_cast<const int32_t*>(tb + to);
+                        zr[i][0] = z[0];
+                        zr[i][1] = z[1];
+                        zk[i] = *(const QG u32_2*)(ob + (uint32_t)oo);
+                    }
+                    if (kCol0) {  // qxa = 0, so xq = x
+                        const uint64_t zc[2] = {__ballot(xq == 0), __ballot(xq + 1 == W)};
+                        if ((zc[0] | zc[1]) != 0ull) {
 #pragma unroll
-                    for (int j = 0; j < SPT; ++j) {
-                        // t = base + u 2048 + j BT + tid = y W + x, slot j BT +
-                        // tid; for t < thi <= T <= 2^23, y < 2^23 fits the
-                        // 24-bit products
-                        int32_t yv = y;
-                        if (kCol0) {
-                            // lanes hold consecutive t: a wave meets x = 0 once
-                            // per W values of t, so the fp32 row is formed only then
-                            const bool z = x == 0;
-                            if (__ballot(z) != 0ull) {
-                                // kept as a branch (not evaluated for every t)
-                                __asm__ volatile("" ::: "memory");
-                                if (z && row_of(y * W, vis.rW) != y) yv = y - 1;
+                            for (int j = 0; j < 2; ++j) {
+                                const int32_t yt = y + j;  // t + j = yt W
+                                const int32_t yv = yt - (row_of(yt * W, vis.rW) != yt ? 1 : 0);
+                                const bool c = j == 0 ? xq == 0 : xq + 1 == W;
+                                const bool q = c && t + j < T && (uint32_t)(yv - ka) < (uint32_t)(kb - ka);
+                                in[i][j] = (in[i][j] & ~zc[j]) | __ballot(q);
+                                if (q) {
+                                    zr[i][j] = tile[(yv + minY - db0) * DW + minX - dx0];
+                                    const uint32_t k = obs[(yv + minY - ry0) * rw + minX - rx0];
+                                    zk[i] = j == 0 ? (zk[i] & 0xffff0000u) | k : (zk[i] & 0xffffu) | (k << 16);
+                                }
                             }
                         }
-                        zr[u][j] = QPSO_EMPTY;
-                        zk[u][j] = 0;
-                        if ((!kLast || (uint32_t)(base + u * 2048 + j * BT + tid) < (uint32_t)thi) &&
-                            (uint32_t)(x - qxa) < xn && (uint32_t)(yv - qya) < yn) {
-                            zr[u][j] = tile[__mul24(yv, DW) + x + tc];
-                            const uint32_t oi = (uint32_t)(__mul24(yv, rw) + x + oc);  // >= 0: a rect pixel
-                            zk[u][j] = (int32_t)*(const QG uint16_t*)(ob + 2u * oi);
-                        }
-                        x += sr;
-                        y += sq;
-                        if (x >= W) { x -= W; ++y; }
                     }
+                    const bool wrap = xq >= xlim;
+                    xq += wrap ? x1s : x0s;
+                    to += wrap ? to1 : to0;
+                    oo += wrap ? oo1 : oo0;
+                    if (kCol0) y += sq + (wrap ? 1 : 0);
                 }
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
+                for (int i = 0; i < U * PR; ++i) {
 #pragma unroll
-                    for (int j = 0; j < SPT; ++j) {
+                    for (int j = 0; j < 2; ++j) {
                         // an empty or unobserved pixel adds fma(0, 0, acc) = acc
                         // (acc >= +0)
-                        const bool r = zr[u][j] != QPSO_EMPTY, o = zk[u][j] != 0;
-                        const uint64_t mr = __ballot(r), mo = __ballot(o);
-                        w_rend += (uint32_t)__popcll(mr);
-                        w_tr += (uint32_t)__popcll(mr & ~mo);
-                        w_seg += (uint32_t)__popcll(mo & ~mr);
-                        const float e = (float)((r && o) ? wsub(zr[u][j], zk[u][j]) : 0) * 0.001f;
-                        acc_e[j] = __builtin_fmaf(e, e, acc_e[j]);
+                        const int32_t z = zr[i][j], k = (int32_t)(j == 0 ? zk[i] & 0xffffu : zk[i] >> 16);
+                        const uint64_t r = __ballot(z != QPSO_EMPTY) & in[i][j], o = __ballot(k != 0) & in[i][j];
+                        w_rend += (uint32_t)__popcll(r);
+                        w_obs += (uint32_t)__popcll(o);
+                        w_both += (uint32_t)__popcll(r & o);
+                        float e = (float)wsub(z, k) * 0.001f;
+                        e = __builtin_amdgcn_inverse_ballot_w64(r & o) ? e : 0.0f;
+                        acc_e[i % PR][j] = __builtin_fmaf(e, e, acc_e[i % PR][j]);
                     }
                 }
             };
             using yes = std::true_type;
             using no = std::false_type;
-            for (int32_t base = (tlo / 2048) * 2048; base < thi; base += 2048 * U) {
-                const bool last = base + 2048 * U > thi;
+            for (int32_t base = base0; base < thi; base += 2048 * U) {
+                const bool edge = base < ta || base + 2048 * U >= thi;
                 if (col0) {
-                    if (last) batch(base, yes{}, yes{});
+                    if (edge) batch(base, yes{}, yes{});
                     else batch(base, yes{}, no{});
                 } else {
-                    if (last) batch(base, no{}, yes{});
+                    if (edge) batch(base, no{}, yes{});
                     else batch(base, no{}, no{});
                 }
             }
             if ((tid & 63) == 0) {
                 n_rend += w_rend;
-                n_tr += w_tr;
-                n_seg += w_seg;
+                n_tr += w_rend - w_both;
+                n_seg += w_obs - w_both;
             }
         }
 
@@ -1187,11 +1217,14 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     }
 
     // ---- reductions (FitnessReductionBallot, main.h:1522-1573): halving tree
-    //      over the 2048 error slots; thread tid holds slots tid + j*BT
+    //      over the 2048 error slots; a thread's pairs lie 2 BT slots apart
 #pragma unroll
-    for (int stride = 1024; stride >= BT; stride >>= 1) {
+    for (int half = PR / 2; half >= 1; half >>= 1) {
 #pragma unroll
-        for (int j = 0; j < stride / BT; ++j) acc_e[j] = acc_e[j] + acc_e[j + stride / BT];
+        for (int i = 0; i < half; ++i) {
+            acc_e[i][0] = acc_e[i][0] + acc_e[i + half][0];
+            acc_e[i][1] = acc_e[i][1] + acc_e[i + half][1];
+        }
     }
     const uint32_t cs = wave_sum(n_seg), ct = wave_sum(n_tr), cr = wave_sum(n_rend);
     if ((tid & 63) == 0) {
@@ -1208,14 +1241,15 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     // then wave 0 runs the rest of the tree: slot t = lane + 64 k sits in
     // v[k], so level "t += t + stride" is v[k] += v[k + stride / 64]
     float* red = reinterpret_cast<float*>(rings);
-    red[tid] = acc_e[0];
+    red[2 * tid] = acc_e[0][0];
+    red[2 * tid + 1] = acc_e[0][1];
     __syncthreads();
     if (tid < 64) {
-        float r[BT / 64];
+        float r[BT / 32];
 #pragma unroll
-        for (int k = 0; k < BT / 64; ++k) r[k] = red[tid + 64 * k];
+        for (int k = 0; k < BT / 32; ++k) r[k] = red[tid + 64 * k];
 #pragma unroll
-        for (int s = BT / 128; s >= 1; s >>= 1) {
+        for (int s = BT / 64; s >= 1; s >>= 1) {
 #pragma unroll
             for (int k = 0; k < s; ++k) r[k] = r[k] + r[k + s];
         }
