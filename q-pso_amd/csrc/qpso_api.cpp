@@ -54,7 +54,7 @@ constexpr size_t kRandIdleBytes = size_t(256) << 20;
 
 struct Mesh {
     float* verts = nullptr;        // unique vertices [3][V]
-    QpsoFaceRef* faces = nullptr;  // interleaved raster order [F]
+    QpsoFaceIdx* faces = nullptr;  // vertex indices per face, face order [F]
     float* corners = nullptr;      // [F][3][4]: a face's corners (x, y, z, vertex index bits), 16 bytes each
     uint32_t F = 0, V = 0;
     std::vector<uint32_t> v_prefix;  // unique vertices referenced by faces [0, f+1)
@@ -540,15 +540,17 @@ int qpso_mesh_upload(qpso_ctx* ctx, const float* soa, uint32_t n_faces, uint32_t
     m.V = (uint32_t)(verts.size() / 3);
     std::vector<float> corners;
     qpso_host::build_corner_table(soa, n_faces, order, corners);
+    std::vector<QpsoFaceIdx> idx;
+    qpso_host::build_index_table(order, idx);
     hipError_t e = hipMalloc(&m.corners, sizeof(float) * corners.size());
     if (e == hipSuccess) e = hipMalloc(&m.verts, sizeof(float) * verts.size());
-    if (e == hipSuccess) e = hipMalloc(&m.faces, sizeof(QpsoFaceRef) * order.size());
+    if (e == hipSuccess) e = hipMalloc(&m.faces, sizeof(QpsoFaceIdx) * idx.size());
     if (e == hipSuccess) e = hipMalloc(&m.runs, sizeof(int32_t) * std::max<size_t>(runs.size(), 1));
     if (e == hipSuccess) e = copy_on(ctx->stream, m.verts, verts.data(), sizeof(float) * verts.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = copy_on(ctx->stream, m.corners, corners.data(), sizeof(float) * corners.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess)
-        e = copy_on(ctx->stream, m.faces, order.data(), sizeof(QpsoFaceRef) * order.size(), hipMemcpyHostToDevice);
+        e = copy_on(ctx->stream, m.faces, idx.data(), sizeof(QpsoFaceIdx) * idx.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess && !runs.empty())
         e = copy_on(ctx->stream, m.runs, runs.data(), sizeof(int32_t) * runs.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {

@@ -43,6 +43,13 @@ struct QpsoFaceRef {
     int32_t v0, v1, v2, face;
 };
 
+// The device's raster table: the indices modulo 65536, eight bytes a face.  A
+// vertex cache holds fewer vertices than that, so an index relative to the
+// cache's first vertex is exact modulo 65536.
+struct QpsoFaceIdx {
+    uint16_t v0, v1, v2, pad;
+};
+
 struct QpsoSolveDev {
     // mesh (metres)
     int32_t F;       // faces
@@ -51,7 +58,7 @@ struct QpsoSolveDev {
     const float* verts;
     int32_t V;       // unique vertices (row stride of verts)
     int32_t V_eff;   // unique vertices referenced by faces < F_eff (a prefix)
-    const QpsoFaceRef* faces;
+    const QpsoFaceIdx* faces;
     const float* corners;  // [F][3][4]: face f's corner j at corners[12 f + 4 j], (x, y, z, vertex index bits)
     int32_t n_faces; // entries in `faces` (= F)
     // runs of consecutive faces whose corners lie in a short vertex range:

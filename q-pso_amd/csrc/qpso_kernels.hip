@@ -25,6 +25,7 @@
 #include "qpso_internal.h"
 #include "qpso_kernels.h"
 #include "qpso_math.h"
+#include "qpso_tables.h"
 
 using namespace qpso;
 
@@ -38,10 +39,8 @@ constexpr int kCols = 640;
 #define QG __attribute__((address_space(1)))
 typedef int32_t qv4 __attribute__((ext_vector_type(4)));
 typedef int32_t qv2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ QpsoFaceRef load_ref(const QG QpsoFaceRef* p, int i) {
-    const qv4 v = reinterpret_cast<const QG qv4*>(p)[i];
-    return QpsoFaceRef{v.x, v.y, v.z, v.w};
-}
+// a face's three vertex indices modulo 65536: x = v0 | v1 << 16, y = v2
+__device__ __forceinline__ qv2 load_ref(const QG QpsoFaceIdx* p, int i) { return reinterpret_cast<const QG qv2*>(p)[i]; }
 __device__ __forceinline__ QpsoStale load_stale(const QG QpsoStale* p, int i) {
     const qv2 v = reinterpret_cast<const QG qv2*>(p)[i];
     return QpsoStale{v.x, v.y};
@@ -50,30 +49,39 @@ __device__ __forceinline__ void store_stale(QG QpsoStale* p, int i, int32_t pos,
     reinterpret_cast<QG qv2*>(p)[i] = qv2{pos, val};
 }
 
+// Reductions over a wave in DPP steps (a lane's neighbours in its row of 16,
+// then the last lanes of rows 0 and 2, then of row 1): the total stands in
+// lane 63 and is read from there into a scalar.  A shuffle through LDS takes
+// about ten times a step's time.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp(int old, int v) {
+    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xf, false);
+}
+template <class F>
+__device__ __forceinline__ int wave_reduce(int v, int id, F f) {
+    v = f(v, dpp<0x111, 0xf>(id, v));  // row_shr:1
+    v = f(v, dpp<0x112, 0xf>(id, v));  // row_shr:2
+    v = f(v, dpp<0x114, 0xf>(id, v));  // row_shr:4
+    v = f(v, dpp<0x118, 0xf>(id, v));  // row_shr:8
+    v = f(v, dpp<0x142, 0xa>(id, v));  // row_bcast:15 into rows 1 and 3
+    v = f(v, dpp<0x143, 0xc>(id, v));  // row_bcast:31 into rows 2 and 3
+    return __builtin_amdgcn_readlane(v, 63);
+}
 __device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
-    return v;
+    return wave_reduce(v, INT32_MAX, [](int a, int b) { return min(a, b); });
 }
 __device__ __forceinline__ int wave_max(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
-    return v;
+    return wave_reduce(v, INT32_MIN, [](int a, int b) { return max(a, b); });
 }
 __device__ __forceinline__ unsigned wave_sum(unsigned v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += (unsigned)__shfl_xor((int)v, o);
-    return v;
+    return (unsigned)wave_reduce((int)v, 0, [](int a, int b) { return (int)((unsigned)a + (unsigned)b); });
 }
-
 __device__ __forceinline__ unsigned long long wave_sum64(unsigned long long v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const unsigned lo = (unsigned)__shfl_xor((int)(unsigned)v, o);
-        const unsigned hi = (unsigned)__shfl_xor((int)(unsigned)(v >> 32), o);
-        v += ((unsigned long long)hi << 32) | lo;
-    }
-    return v;
+    // four sums of 16-bit parts fit 22 bits each
+    const unsigned a = wave_sum((unsigned)(v & 0xffffu)), b = wave_sum((unsigned)((v >> 16) & 0xffffu));
+    const unsigned c = wave_sum((unsigned)((v >> 32) & 0xffffu)), d = wave_sum((unsigned)(v >> 48));
+    return (unsigned long long)a + ((unsigned long long)b << 16) + ((unsigned long long)c << 32) +
+           ((unsigned long long)d << 48);
 }
 
 #define RT(S, p, s) (S).rand[(size_t)(p) + (size_t)(s) * (size_t)(S).N]
@@ -155,6 +163,42 @@ struct Visits {
 // and 128 registers, which its bodies exceed without spilling at 3.
 constexpr int rf_waves_per_simd(int bt, int cap) {
     return bt >= 512 ? (bt / 256) * ((160 * 1024) / (cap * 4 + 512)) : 1;
+}
+
+typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_xy(int32_t X, int32_t Y) {  // X | Y << 16 (low halves)
+    return __builtin_amdgcn_perm((uint32_t)Y, (uint32_t)X, 0x05040100u);
+}
+// The cull's test of a face with packed corners (28.4, 16-bit halves whose
+// differences fit 16 bits, |a| <= 32767 - 15): front-facing, non-empty and
+// overlapping the region from lo (x | y << 16, inclusive) to hi (exclusive).
+// keep: it starts above row b1; down: it ends below it (b1w = b1 << 16; the y
+// half decides a 32-bit comparison against it).  20 instructions instead of 48
+// on 32-bit coordinates.
+__device__ __forceinline__ bool cull_packed(uint32_t pa, uint32_t pb, uint32_t pc, uint32_t lo, uint32_t hi,
+                                            int32_t b1w, bool& keep, bool& down) {
+    const i16x2 A = __builtin_bit_cast(i16x2, pa), B = __builtin_bit_cast(i16x2, pb), C = __builtin_bit_cast(i16x2, pc);
+    const i16x2 c15 = {15, 15}, c4 = {4, 4}, c1 = {1, 1};
+    const i16x2 mn = (__builtin_elementwise_min(__builtin_elementwise_min(A, B), C) + c15) >> c4;
+    const i16x2 mx = (__builtin_elementwise_max(__builtin_elementwise_max(A, B), C) + c15) >> c4;
+    const i16x2 d = __builtin_elementwise_min(mx, __builtin_bit_cast(i16x2, hi)) -
+                    __builtin_elementwise_max(mn, __builtin_bit_cast(i16x2, lo));
+    const bool in = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(d, c1)) == 0x00010001u;
+    const int32_t ab = __builtin_bit_cast(int32_t, A - B), ca = __builtin_bit_cast(int32_t, C - A);
+    // DX12 DY31 > DX31 DY12: both products below 2^30
+    const bool front = __mul24((ab << 16) >> 16, ca >> 16) > __mul24((ca << 16) >> 16, ab >> 16);
+    keep = __builtin_bit_cast(int32_t, mn) < b1w;
+    down = __builtin_bit_cast(int32_t, mx) > (b1w | 0xffff);
+    return in && front;
+}
+__device__ __forceinline__ void todo_mask(uint64_t todo, bool reach, bool keep, bool down, uint64_t& m, uint64_t& lm) {
+    const uint64_t r = todo & __ballot(reach);
+    m = r & __ballot(keep);
+    lm = r & __ballot(down);
+}
+__device__ __forceinline__ uint64_t uniform64(uint64_t v) {  // a wave-uniform value into scalar registers
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+           (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
 }
 
 // The render kernel's LDS, declared once per kernel and shared by the bodies
@@ -250,7 +294,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
 
     const Cam cam{S.fx, S.fy, S.cx, S.cy};
     const int Fe = S.F_eff;
-    const QG QpsoFaceRef* __restrict__ faces = (const QG QpsoFaceRef*)S.faces;
+    const QG QpsoFaceIdx* __restrict__ faces = (const QG QpsoFaceIdx*)S.faces;
     const int n_faces = S.n_faces;
     const int32_t big_face = S.big_face;
 
@@ -266,37 +310,43 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     }
     __syncthreads();
 
-    // The projected unique vertices of a mesh of at most kWin vertices stay in
-    // LDS.  A larger mesh is cut on the host into runs of faces whose corners
-    // lie in a short range of vertex indices; each band then takes the runs
-    // in windows (consecutive runs whose joint range fits the cache) and
-    // projects the windows in turn.  Without usable runs every face's corners
-    // are projected where needed.
-    //   A vertex takes three words, X and Y read together, then Z; or, packed,
-    // one word, X and Y as 16-bit halves, and a drawn face's corner depths
-    // are projected again from the face's corner table.  Packing gives the
-    // tile two words per vertex for that re-projection.  It is taken when
-    // every 28.4 coordinate of the particle fits the halves (checked after
-    // pass A) and, for a cached mesh, a depth region covering the whole
-    // cluster rect would not fit beside the three-word cache in one band.
-    // Windows always pack: a window then holds 2 kWin vertices and the tile
-    // gains kWin words, and a face's cull reads one word per corner (measured
-    // faster even where the band count stays the same).
-    const bool cached = !WIN || Ve <= kWin;  // compile-time true without windows
-    const bool runs = WIN && !cached && S.n_runs > 0 && S.n_runs * 256 <= Fe;  // runs of 256 faces on average
-    int VC = cached ? Ve : (runs ? kWin : 0);  // cache capacity in vertices (three-word)
+    // The projected unique vertices stay in LDS, one word each: X and Y in 28.4
+    // as 16-bit halves, which the cull reads with packed 16-bit instructions.
+    // With room beside a depth region covering the whole cluster rect, a
+    // second word holds Z (zc); otherwise a drawn face's corner depths are
+    // projected again from the face's corner table.  A particle with vertices
+    // beyond the halves, or a box too wide for their differences, projects
+    // every face from the corner table instead (pack = false).
+    //   Any mesh is kept whole (cached) that leaves the rect a depth region of
+    // half its size, or that is no larger than the packed window of kWin words
+    // twice.  A larger one is cut on the host into runs of faces whose
+    // corners lie in a short range of vertex indices; each band then takes
+    // the runs in windows (consecutive runs whose joint range fits the cache)
+    // and projects the windows in turn.  Without usable runs every face is
+    // projected from the corner table.
     constexpr int kQCap = CAP / 32;   // small faces needing the per-pixel depth
     constexpr int kBQCap = CAP / 128;
-    constexpr int kRing = 128;
+    // batches of 64 faces culled together between draws: their latencies
+    // overlap, at the price of empty ones at a mesh's end.  The 10k-face
+    // mesh has ten a wave: 151k clocks a workgroup with 1, 156k with 2; the
+    // 50k-face one 174k with 1, 167k with 2 (3 spills registers).
+    constexpr int kGroup = WIN ? 2 : 1;
+    constexpr int kRing = 64 * (kGroup + 1);
     constexpr int kFixed = kQCap + 4 * kBQCap + (BT / 64) * kRing + 4;  // queues, rings, alignment
-    bool pack = runs;
-    if (cached) {
+    constexpr int kMinVC = CAP / 12 > qpso_host::kRunVerts ? CAP / 12 : qpso_host::kRunVerts;  // shortest window
+    constexpr int kMinTile = 2048 + CAP / 8;  // a row of the frame with its lines, and the later bits
+    const int32_t rect_words = [&] {  // a band of the whole rect
         const int32_t rw = S.rect[2] - S.rect[0], rh = S.rect[3] - S.rect[1];
-        pack = rw * rh + rh * (((rw + 31) >> 5) + 1) + rw + 8 > CAP - kFixed - 3 * VC;
-    }
-    uint32_t* __restrict__ vP = reinterpret_cast<uint32_t*>(lds);  // packed: X | Y << 16
-    int2* __restrict__ vXY = reinterpret_cast<int2*>(lds);  // X, Y in one 8-byte read
-    float* __restrict__ vZ = reinterpret_cast<float*>(lds + 2 * VC);  // set again below for windows
+        return rw * rh + rh * (((rw + 31) >> 5) + 1) + rw + 8;
+    }();
+    // compile-time true without windows
+    const bool cached = !WIN || Ve <= max(2 * kWin, CAP - kFixed - max(rect_words / 2 + 1024, kMinTile));
+    const bool runs = WIN && !cached && S.n_runs > 0 && S.n_runs * 256 <= Fe;  // runs of 256 faces on average
+    bool pack = cached || runs;
+    int VC = cached ? Ve : 2 * kWin;  // cache capacity in vertices
+    const bool zc = cached && max(rect_words, kMinTile) <= CAP - kFixed - 2 * VC;
+    uint32_t* __restrict__ vP = reinterpret_cast<uint32_t*>(lds);  // X | Y << 16
+    float* __restrict__ vZ = reinterpret_cast<float*>(lds + VC);
     int32_t vbase = 0;  // vertex index of cache entry 0
     // windows: the vertices [cbase, chi) the cache holds projected (entry
     // v - cbase), so that a window inside them is not projected again
@@ -317,13 +367,10 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             auto take = [&](int v, float x, float y, float z) {
                 int32_t X, Y;
                 float Z;
-                dg |= vertex_fixed(pose, x, y, z, cam, X, Y, Z) ? 1 : 0;
-                if (cached) {
-                    if (pack) vP[v] = ((uint32_t)X & 0xffffu) | ((uint32_t)Y << 16);  // used only if all fit
-                    else { vXY[v] = make_int2(X, Y); vZ[v] = Z; }
-                } else if (runs && v < 2 * kWin) {
-                    // the packed window from vertex 0, kept if every coordinate fits
-                    vP[v] = ((uint32_t)X & 0xffffu) | ((uint32_t)Y << 16);
+                vertex_fixed(pose, x, y, z, cam, X, Y, Z);
+                if (!WIN || v < VC) {  // windows: the one from vertex 0, kept if every coordinate fits
+                    if (pack) vP[v] = pack_xy(X, Y);
+                    if (zc) vZ[v] = Z;
                 }
                 xl = min(xl, X); xh = max(xh, X);
                 yl = min(yl, Y); yh = max(yh, Y);
@@ -338,6 +385,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             if (xl <= xh) {
                 bx0 = min(bx0, wadd(xl, 15) >> 4); bx1 = max(bx1, wadd(xh, 15) >> 4);
                 by0 = min(by0, wadd(yl, 15) >> 4); by1 = max(by1, wadd(yh, 15) >> 4);
+                dg = beyond_limit(xl, xh, yl, yh);
             }
         }
         bx0 = wave_min(bx0); bx1 = wave_max(bx1);
@@ -373,46 +421,10 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     }
 
     // (X + 15) >> 4 >= -2047 gives X >= -32767 and <= 2046 gives X <= 32736:
-    // every cached vertex fits the 16-bit halves.  A particle with vertices
-    // beyond them writes the three-word cache instead (its vertices are still
-    // in registers; the packed words are never read) and takes more bands;
-    // with windows it projects them in three words.
-    if (pack && !(ax0 >= -2047 && ax1 <= 2046 && ay0 >= -2047 && ay1 <= 2046)) {
+    // every cached vertex fits the 16-bit halves; a box of at most 2046 pixels
+    // a side keeps their differences and (a + 15) in 16 bits too
+    if (!(ax0 >= -2047 && ax1 <= 2046 && ay0 >= -2047 && ay1 <= 2046 && ax1 - ax0 <= 2046 && ay1 - ay0 <= 2046))
         pack = false;
-#pragma unroll
-        for (int j = 0; j < kVPT; ++j) {
-            const int v = tid + j * BT;
-            if (cached && v < Ve) {
-                int32_t X, Y;
-                float Z;
-                vertex_fixed(pose, ux[j], uy[j], uz[j], cam, X, Y, Z);
-                vXY[v] = make_int2(X, Y);
-                vZ[v] = Z;
-            }
-        }
-    }
-    // queue of small faces needing the per-pixel depth (kQCap entries); big
-    // faces of more than S.big_face pixels (non-flat ones: half as many),
-    // rasterized by a whole wave so one large face does not hold its wave's
-    // other 63 lanes idle: clipped
-    // rectangle (x0 | x1 << 16, y0 | y1 << 16), constant depth, face << 1 | flat
-    if (WIN && runs) {  // window capacity in vertices
-        VC = pack ? 2 * kWin : kWin;
-        vZ = reinterpret_cast<float*>(lds + 2 * VC);
-        if (pack) chi = min(Ve, 2 * kWin);  // pass A's window [0, chi)
-    }
-    int32_t* __restrict__ queue = lds + (pack ? VC : 3 * VC);
-    int32_t* __restrict__ bq_x = queue + kQCap;
-    int32_t* __restrict__ bq_y = bq_x + kBQCap;
-    int32_t* __restrict__ bq_k = bq_y + kBQCap;
-    int32_t* __restrict__ bq_i = bq_k + kBQCap;
-    // per wave: ring of kRing culled face entries waiting to be drawn
-    int32_t* __restrict__ rings = bq_i + kBQCap;
-    // the tile starts on a 16-byte boundary for 128-bit fills
-    const int32_t tile_off = (int32_t)(rings - lds) + (BT / 64) * kRing;
-    int32_t* __restrict__ tile = lds + ((tile_off + 3) & ~3);
-    const int32_t tcap = CAP - ((tile_off + 3) & ~3);
-
     const int32_t W = (int32_t)W64, H = (int32_t)H64;
     const int32_t A = W * H;
     const int32_t T = ((A + 1023) >> 10) << 10;  // NumIters * 1024 (main.cu:621-623)
@@ -421,8 +433,9 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     const int32_t rw = rx1 - rx0;
     const QG uint16_t* __restrict__ obs = (const QG uint16_t*)S.obs;
 
-    // carried pixels inside the union box join the tile region
-    {
+    // carried pixels inside the union box join the tile region (n_old is
+    // uniform; without any, s_stale stays empty)
+    if (n_old > 0) {
         int32_t sx0 = INT32_MAX, sx1 = INT32_MIN, sy0 = INT32_MAX, sy1 = INT32_MIN;
 #pragma unroll
         for (int j = 0; j < kSPT; ++j) {
@@ -434,16 +447,14 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                 sy0 = min(sy0, ey); sy1 = max(sy1, ey);
             }
         }
-        if (n_old > 0) {
-            sx0 = wave_min(sx0); sx1 = wave_max(sx1);
-            sy0 = wave_min(sy0); sy1 = wave_max(sy1);
-            if ((tid & 63) == 0 && sx0 <= sx1) {
-                atomicMin(&s_stale[0], sx0); atomicMax(&s_stale[1], sx1);
-                atomicMin(&s_stale[2], sy0); atomicMax(&s_stale[3], sy1);
-            }
+        sx0 = wave_min(sx0); sx1 = wave_max(sx1);
+        sy0 = wave_min(sy0); sy1 = wave_max(sy1);
+        if ((tid & 63) == 0 && sx0 <= sx1) {
+            atomicMin(&s_stale[0], sx0); atomicMax(&s_stale[1], sx1);
+            atomicMin(&s_stale[2], sy0); atomicMax(&s_stale[3], sy1);
         }
+        __syncthreads();
     }
-    __syncthreads();
     // Tile region: rendered AABB plus those carried pixels, inside the frame.
     // Every depth value other than 60000 in the union box lies in it.
     int32_t tx0 = ax0, tx1 = ax1, ty0 = ay0, ty1 = ay1;  // [x0, x1) x [y0, y1)
@@ -469,6 +480,46 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     const int32_t MW = full ? 0 : (TW + 31) >> 5;  // mask words per tile row
     const bool col_line = minX >= tx0 && minX < tx1;
 
+    // ---- LDS: [vertex cache] [queues] [rings] [later bits] [tile]
+    // words of a band of the whole region; `later` bits only where that does
+    // not fit beside the rest
+    const int32_t TH = has_tile ? ty1 - ty0 : 0;
+    const int32_t region = TH * (MW + 1) + (DW > 0 ? DW * (dy1 - dy0) : 0);
+    const int32_t n_lw = (Fe + 63) >> 6;
+    const bool win = WIN && runs && pack;
+    int32_t v_words = !pack ? 0 : zc ? 2 * VC : VC;
+    bool lbits = region + TW + 8 > CAP - kFixed - (win ? kMinVC : v_words);
+    lbits = lbits && 2 * n_lw <= CAP / 8;
+    if (win) {
+        // the largest window, up to 2 kWin, that costs no band: projecting
+        // and culling a band's windows again costs more than shorter windows
+        const int32_t room = CAP - kFixed - (lbits ? 2 * n_lw : 0) - TW - 8;
+        int32_t vw = room - region;
+        for (int32_t nb = 2; vw < kMinVC && nb <= 16; ++nb) vw = room - (region + nb - 1) / nb - DW - MW - 1;
+        VC = min(2 * kWin, max(vw, kMinVC));
+        chi = min(min(Ve, 2 * kWin), VC);  // pass A's window [0, chi)
+        v_words = VC;
+    }
+    // queue of small faces needing the per-pixel depth (kQCap entries); big
+    // faces of more than S.big_face pixels (non-flat ones: half as many),
+    // rasterized by a whole wave so one large face does not hold its wave's
+    // other 63 lanes idle: clipped
+    // rectangle (x0 | x1 << 16, y0 | y1 << 16), constant depth, face << 1 | flat
+    int32_t* __restrict__ queue = lds + v_words;
+    int32_t* __restrict__ bq_x = queue + kQCap;
+    int32_t* __restrict__ bq_y = bq_x + kBQCap;
+    int32_t* __restrict__ bq_k = bq_y + kBQCap;
+    int32_t* __restrict__ bq_i = bq_k + kBQCap;
+    // per wave: ring of kRing culled face entries waiting to be drawn
+    int32_t* __restrict__ rings = bq_i + kBQCap;
+    // the later bits on an 8-byte boundary, the tile on a 16-byte one for
+    // 128-bit fills
+    const int32_t l_off = ((int32_t)(rings - lds) + (BT / 64) * kRing + 1) & ~1;
+    unsigned long long* const later = reinterpret_cast<unsigned long long*>(lds + l_off);
+    const int32_t tile_off = (l_off + (lbits ? 2 * n_lw : 0) + 3) & ~3;
+    int32_t* __restrict__ tile = lds + tile_off;
+    const int32_t tcap = CAP - tile_off;
+
     float acc_e[PR][2];  // [i][j]: slot 2 (tid + i BT) + j
 #pragma unroll
     for (int i = 0; i < PR; ++i) acc_e[i][0] = acc_e[i][1] = 0.0f;
@@ -480,44 +531,28 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         if (k < cap) store_stale(nw, k, (y << 16) | x, v);
         else atomicOr(S.flags, QPSO_FLAG_STALE_OVERFLOW);
     };
-    // the face's 28.4 vertices: from the LDS vertex cache, or projected again.
-    // f is the face's index, e its table entry (the host keeps the table in
-    // face order, e.face == f; passing f lets the corner reads go out without
-    // waiting for the entry)
-    auto load_face = [&](int32_t f, const QpsoFaceRef& e, Face& fc) {
-        if (pack) {
-            const int32_t vb = WIN ? vbase : 0;
-            const uint32_t pa = vP[e.v0 - vb], pb = vP[e.v1 - vb], pc = vP[e.v2 - vb];
-            fc.X[0] = (int32_t)(pa << 16) >> 16; fc.Y[0] = (int32_t)pa >> 16;
-            fc.X[1] = (int32_t)(pb << 16) >> 16; fc.Y[1] = (int32_t)pb >> 16;
-            fc.X[2] = (int32_t)(pc << 16) >> 16; fc.Y[2] = (int32_t)pc >> 16;
-            // corner depths: pass A's projection of the same coordinates,
-            // read as one 16-byte entry per corner
-            typedef float f4 __attribute__((ext_vector_type(4)));
-            const QG f4* __restrict__ cr = (const QG f4*)S.corners + 3 * (size_t)f;
+    // a face to draw: X and Y from the vertex cache, Z from there too or
+    // projected again from the corner table (pass A's projection of the same
+    // coordinates, one 16-byte entry per corner, which carries the vertex
+    // index: the face table entry is not read); or all three projected
+    // again (in_cache false: the same arithmetic, so the same bits)
+    bool in_cache = pack;
+    auto draw_face = [&](int32_t f, Face& fc) {
+        if (!in_cache) {
+            face_project(S.corners, f, pose, cam, fc);
+            return;
+        }
+        if (zc) {
+            const qv2 e = load_ref(faces, f);
+            const int32_t v[3] = {e.x & 0xffff, (int32_t)((uint32_t)e.x >> 16), e.y & 0xffff};
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                const f4 c = cr[j];
-                float u, v;
-                project(pose, c.x, c.y, c.z, cam, u, v, fc.Z[j]);
+                const uint32_t w = vP[v[j]];
+                fc.X[j] = (int32_t)(w << 16) >> 16;
+                fc.Y[j] = (int32_t)w >> 16;
+                fc.Z[j] = vZ[v[j]];
             }
-            face_bbox(fc);
-        } else if (!WIN || VC > 0) {  // always cached without windows
-            const int32_t vb = WIN ? vbase : 0;
-            const int32_t a = e.v0 - vb, b = e.v1 - vb, c = e.v2 - vb;
-            const int2 pa = vXY[a], pb = vXY[b], pc = vXY[c];
-            fc.X[0] = pa.x; fc.Y[0] = pa.y; fc.Z[0] = vZ[a];
-            fc.X[1] = pb.x; fc.Y[1] = pb.y; fc.Z[1] = vZ[b];
-            fc.X[2] = pc.x; fc.Y[2] = pc.y; fc.Z[2] = vZ[c];
-            face_bbox(fc);
         } else {
-            face_project(S.corners, e.face, pose, cam, fc);
-        }
-    };
-    // a face to draw: with the packed cache its corner entries carry the
-    // vertex indices (w), so the face table entry is not read
-    auto draw_face = [&](int32_t f, Face& fc) {
-        if (pack) {
             typedef float f4 __attribute__((ext_vector_type(4)));
             const QG f4* __restrict__ cr = (const QG f4*)S.corners + 3 * (size_t)f;
             const int32_t vb = WIN ? vbase : 0;
@@ -534,13 +569,10 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                 float u, v;
                 project(pose, c.x, c.y, c.z, cam, u, v, fc.Z[j]);
             }
-            face_bbox(fc);
-        } else {
-            load_face(f, load_ref(faces, f), fc);
         }
+        face_bbox(fc);
     };
-    // a queued face, drawn after its window (windowed meshes: projected from
-    // the corner table, the same arithmetic as the cache's, so the same bits)
+    // a queued face, drawn after its window
     auto queued_face = [&](int32_t f, Face& fc) {
         if (WIN && runs) face_project(S.corners, f, pose, cam, fc);
         else draw_face(f, fc);
@@ -698,20 +730,23 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             return y >= y_end;
         };
         if (take(min(dy0, ty1), cr) && take(DW > 0 ? dy1 : y, cr + DW)) take(ty1, cr);
-        return max(y, b0 + 1);  // one D row fits: TW <= 640 and tcap >= 3909
+        return max(y, b0 + 1);  // one D row fits: TW <= 640 and tcap >= 2048
     };
 
     uint32_t* mask = nullptr;    // [band rows][MW]
     int32_t* col_d = nullptr;    // [band rows]: depth of (minX, y)
     int32_t* row_d = nullptr;    // [TW]: depth of (x, maxY)
-    uint64_t fmask = ~0ull;  // bit k: face entry tid + k*BT still reaches later bands (meshes without windows)
-    const bool use_mask = !runs && n_faces <= 64 * BT;
-    // windows: bit w, window w of a band (the same windows every band) still
-    // has faces reaching later bands; a window without is neither projected
-    // nor culled again.  wslot: the windows drawn so far mod 3, the slot of
-    // s_later the current window uses.
+    // A region of several bands: bit f of `later`, face f is front-facing and
+    // reaches rows below the band, set while a band culls; the next band
+    // takes only those faces.  With windows a later band draws them straight
+    // from the corner table (no window is projected or culled again); without
+    // the bits (more faces than kLater words hold) it culls every window again
+    // but those none of whose faces reached later rows (bit w of wmask; wslot:
+    // the windows drawn so far mod 3, the slot of s_later the current one
+    // uses).
     uint64_t wmask = ~0ull;
     int wslot = 0;
+    bool first = true;
     for (int32_t b0 = ty0, b1; has_tile && b0 < ty1; b0 = b1) {
         b1 = band_end(b0);  // band rows [b0, b1)
         const int32_t nb = b1 - b0;
@@ -722,6 +757,9 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         col_d = reinterpret_cast<int32_t*>(mask) + nb * MW;
         row_d = col_d + nb;
         const bool row_line = maxY >= b0 && maxY < b1;
+        const bool more = b1 < ty1;  // bands follow
+        if (lbits && first && more)
+            for (int i = tid; i < n_lw; i += BT) later[i] = 0ull;
         {
             typedef int32_t v4i __attribute__((ext_vector_type(4)));
             v4i* t4 = reinterpret_cast<v4i*>(tile);
@@ -733,6 +771,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         }
         __syncthreads();
         // pixels carried over from earlier iterations (their values are below 60000)
+        if (n_old > 0) {
 #pragma unroll
         for (int j = 0; j < kSPT; ++j) {
             if (tid + j * BT >= n_old) break;
@@ -746,6 +785,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             }
         }
         __syncthreads();
+        }
 
         // bits of the mask row y over columns [x0, x1)
         auto mark_rows = [&](int32_t x0, int32_t x1, int32_t y0, int32_t y1) {
@@ -773,6 +813,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         //      and rasterized with the per-pixel depth after the pass; D parts
         //      of more than big_face pixels (non-flat: big_face / 2) go to the
         //      wave queue.
+        const int lane = tid & 63;
         auto draw = [&](int32_t i) {
             Face fc;
             Setup su;
@@ -780,6 +821,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             face_setup(fc, su);
             const int32_t x0 = max(fc.minx, tx0), x1 = min(fc.maxx, tx1);
             const int32_t y0 = max(fc.miny, b0), y1 = min(fc.maxy, b1);
+            if (y0 >= y1) return;  // (later bits not tested) starts below the band
             px_r += (unsigned long long)((x1 - x0) * (y1 - y0));
             // part in D
             const int32_t px0 = max(x0, dx0), px1 = min(x1, dx1), py0 = max(y0, db0), py1 = min(y1, db1);
@@ -823,19 +865,26 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                 bq_k[qb] = kd;
                 bq_i[qb] = (i << 1) | (flat ? 1 : 0);
             } else if (flat && !big) {
-                // rows in chunks of four pixels; a chunk's positions past the
-                // row's end repeat its last pixel (the same minimum again)
-                int32_t* row = tile + __mul24(py0 - db0, DW) + (px0 - dx0);
-                const int32_t last = w - 1;
+                // rows in chunks of four pixels, the last one of a row moved left
+                // to end with it; a row of fewer than four repeats its last
+                // pixel (the same minimum again)
+                // Odd lanes go upwards: the two triangles of a quad, neighbours in
+                // the wave, cover much the same pixels and would meet at each.
+                const bool up = lane & 1;
+                int32_t* row = tile + __mul24((up ? py1 - 1 : py0) - db0, DW) + (px0 - dx0);
+                const int32_t rstep = up ? -DW : DW;
+                const int32_t last = w - 1, end = max(w - 4, 0);
+                const int32_t o1 = min(1, last), o2 = min(2, last), o3 = min(3, last);
                 int32_t c = 0, rows = py1 - py0;
                 while (rows > 0) {
-                    atomicMin(row + c, kd);
-                    atomicMin(row + min(c + 1, last), kd);
-                    atomicMin(row + min(c + 2, last), kd);
-                    atomicMin(row + min(c + 3, last), kd);
+                    int32_t* const a = row + min(c, end);
+                    atomicMin(a, kd);
+                    atomicMin(a + o1, kd);
+                    atomicMin(a + o2, kd);
+                    atomicMin(a + o3, kd);
                     c += 4;
                     const bool next = c > last;
-                    row += next ? DW : 0;
+                    row += next ? rstep : 0;
                     rows -= next ? 1 : 0;
                     c = next ? 0 : c;
                 }
@@ -846,13 +895,18 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             }
         };
         int32_t* __restrict__ ring = rings + (tid >> 6) * kRing;
-        const int lane = tid & 63;
-        const uint64_t below = (1ull << lane) - 1ull;
+        // a later band draws the faces of the later bits; it tests them (and
+        // updates the bits) where a band follows and the cache holds them
+        const bool direct = !first && lbits && !(cached && more);
+        in_cache = pack && (cached || !direct);
+        // packed bounds of the band's part of the tile: x | y << 16
+        const uint32_t lo2 = (uint32_t)tx0 | ((uint32_t)b0 << 16), hi2 = (uint32_t)tx1 | ((uint32_t)ty1 << 16);
+        const int32_t b1w = (int32_t)((uint32_t)b1 << 16);
         int run = 0;  // next run of faces (windowed meshes)
         int wi = -1;  // window index in this band
         for (;;) {
-        int f_lo = 0, f_hi = n_faces;
-        if (runs) {
+        int f_lo = 0, f_hi = Fe;
+        if (win && !direct) {
             // the runs whose joint vertex window fits the cache; project it
             const int32_t* __restrict__ rt = S.runs;
             int32_t vlo = rt[3 * run + 1], vhi = rt[3 * run + 2];
@@ -863,7 +917,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                 vhi = max(vhi, rt[3 * r2 + 2]);
                 ++r2;
             }
-            f_hi = r2 < S.n_runs ? rt[3 * r2] : n_faces;
+            f_hi = r2 < S.n_runs ? min(rt[3 * r2], Fe) : Fe;
             run = r2;
             vbase = vlo;
             ++wi;
@@ -881,57 +935,128 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                     int32_t X, Y;
                     float Z;
                     vertex_fixed(pose, wx[v], wy[v], wz[v], cam, X, Y, Z);
-                    if (pack) vP[v - vlo] = ((uint32_t)X & 0xffffu) | ((uint32_t)Y << 16);
-                    else { vXY[v - vlo] = make_int2(X, Y); vZ[v - vlo] = Z; }
+                    vP[v - vlo] = pack_xy(X, Y);
                 }
                 cbase = vlo;
                 chi = vhi;
                 __syncthreads();
             }
         }
-        int head = 0, cnt = 0;  // wave-uniform ring state
-        int k = 0;
-        QpsoFaceRef nxt{0, 0, 0, INT32_MAX};
-        if (f_lo + tid < f_hi) nxt = load_ref(faces, f_lo + tid);
-        if (runs) fmask = 0ull;  // windows: non-zero once a face of the window reaches later bands
-        for (int base = f_lo + tid - lane; base < f_hi; base += BT, ++k) {
-            const int i = base + lane;  // = f_lo + tid + k * BT
-            const QpsoFaceRef e = nxt;  // prefetched one iteration ahead
-            if (i + BT < f_hi) nxt = load_ref(faces, i + BT);
-            bool keep = false;
-            if (i < f_hi && (!use_mask || ((fmask >> k) & 1ull))) {
-                bool later = false;
-                if (e.face < Fe) {
-                    Face fc;
-                    load_face(i, e, fc);
-                    if (max(fc.minx, tx0) < min(fc.maxx, tx1) && fc.miny < ty1 && fc.maxy > b0 && face_front(fc)) {
-                        later = fc.maxy > b1;
-                        keep = fc.miny < b1;
+        // 64 faces at a time; a batch starts on a multiple of 64 so that it
+        // is one word of the later bits.  kGroup batches are culled together,
+        // the face entries of the next group in flight (lanes outside the
+        // window load one of the window's): with one batch in flight the
+        // loads' latency set the pace of the cull.
+        int cnt = 0;  // faces waiting in the ring (wave-uniform), last in first out
+        uint64_t any_later = 0;
+        int base = __builtin_amdgcn_readfirstlane((f_lo & ~63) + tid - lane);
+        const bool fetch = pack && (first || !lbits);  // every face of [f_lo, f_hi), from the cache
+        qv2 nx[kGroup];
+#pragma unroll
+        for (int g = 0; g < kGroup; ++g) nx[g] = qv2{0, 0};
+        if (fetch) {
+#pragma unroll
+            for (int g = 0; g < kGroup; ++g) nx[g] = load_ref(faces, min(max(base + g * BT + lane, f_lo), f_hi - 1));
+        }
+        for (;; base += kGroup * BT) {
+            // per batch of the group: the faces to draw in this band, and
+            // those that reach below it
+            uint64_t m[kGroup], lm[kGroup];
+            if (fetch) {
+                // no test between the batches: their vertex reads and
+                // arithmetic interleave
+                const uint32_t vb = WIN ? (uint32_t)vbase : 0u;
+                uint32_t pv[kGroup][3];
+#pragma unroll
+                for (int g = 0; g < kGroup; ++g) {
+                    const uint32_t x = (uint32_t)nx[g].x, y = (uint32_t)nx[g].y;
+                    pv[g][0] = vP[(x - vb) & 0xffffu];
+                    pv[g][1] = vP[((x >> 16) - vb) & 0xffffu];
+                    pv[g][2] = vP[(y - vb) & 0xffffu];
+                }
+                if (base + kGroup * BT < f_hi) {
+#pragma unroll
+                    for (int g = 0; g < kGroup; ++g) nx[g] = load_ref(faces, min(base + (kGroup + g) * BT + lane, f_hi - 1));
+                }
+#pragma unroll
+                for (int g = 0; g < kGroup; ++g) {
+                    const int i = base + g * BT + lane;
+                    bool keep, down;
+                    const bool reach = cull_packed(pv[g][0], pv[g][1], pv[g][2], lo2, hi2, b1w, keep, down);
+                    const uint64_t in = __ballot((uint32_t)(i - f_lo) < (uint32_t)(f_hi - f_lo)) & __ballot(reach);
+                    m[g] = in & __ballot(keep);
+                    lm[g] = in & __ballot(down);
+                }
+            } else {
+#pragma unroll 1
+                for (int g = 0; g < kGroup; ++g) {
+                    const int bg = base + g * BT, i = bg + lane;
+                    uint64_t mg = 0, lg = 0;
+                    const uint64_t todo = bg >= f_hi ? 0ull : first || !lbits ? ~0ull : uniform64(later[bg >> 6]);
+                    if (direct) {
+                        mg = todo;
+                    } else if (todo != 0ull) {
+                        bool reach = false, keep = false, down = false;
+                        if (i >= f_lo && i < f_hi) {
+                            if (pack) {
+                                const uint32_t vb = WIN ? (uint32_t)vbase : 0u;
+                                const qv2 e = load_ref(faces, i);
+                                const uint32_t x = (uint32_t)e.x, y = (uint32_t)e.y;
+                                reach = cull_packed(vP[(x - vb) & 0xffffu], vP[((x >> 16) - vb) & 0xffffu],
+                                                    vP[(y - vb) & 0xffffu], lo2, hi2, b1w, keep, down);
+                            } else {
+                                Face fc;
+                                face_project(S.corners, i, pose, cam, fc);
+                                reach = max(fc.minx, tx0) < min(fc.maxx, tx1) && fc.miny < ty1 && fc.maxy > b0 && face_front(fc);
+                                keep = fc.miny < b1;
+                                down = fc.maxy > b1;
+                            }
+                        }
+                        todo_mask(todo, reach, keep, down, mg, lg);
+                    }
+                    // (kept in registers indexed at compile time)
+#pragma unroll
+                    for (int k = 0; k < kGroup; ++k) {
+                        if (k == g) { m[k] = mg; lm[k] = lg; }
                     }
                 }
-                if (use_mask && !later) fmask &= ~(1ull << k);
-                if (runs && later) fmask = 1ull;
             }
-            const uint64_t m = __ballot(keep);
-            if (keep) ring[(head + cnt + __popcll(m & below)) & (kRing - 1)] = i;
-            cnt += __popcll(m);
+            if (more) {
+#pragma unroll
+                for (int g = 0; g < kGroup; ++g) {
+                    any_later |= lm[g];
+                    if (lbits && !direct && base + g * BT < f_hi && lane == 0) {
+                        // a window's first and last word is shared with its neighbours
+                        if (!first) later[(base + g * BT) >> 6] = lm[g];
+                        else if (lm[g] != 0ull) atomicOr(&later[(base + g * BT) >> 6], (unsigned long long)lm[g]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < kGroup; ++g) {
+                if (__builtin_amdgcn_inverse_ballot_w64(m[g]))
+                    ring[__builtin_amdgcn_mbcnt_hi((uint32_t)(m[g] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[g], (uint32_t)cnt))] =
+                        base + g * BT + lane;
+                cnt += __popcll(m[g]);
+            }
             __builtin_amdgcn_wave_barrier();
-            if (cnt >= 64) {
-                draw(ring[(head + lane) & (kRing - 1)]);
-                head = (head + 64) & (kRing - 1);
-                cnt -= 64;
+            const bool last = base + kGroup * BT >= f_hi;
+            while (cnt >= 64 || (last && cnt > 0)) {
+                const int n = min(cnt, 64);
+                cnt -= n;
+                if (lane < n) draw(ring[cnt + lane]);
                 __builtin_amdgcn_wave_barrier();
             }
+            if (last) break;
         }
-        if (lane < cnt) draw(ring[(head + lane) & (kRing - 1)]);
-        if (!runs) break;  // one pass over the faces; the queues follow
+        if (!win || direct) break;  // one pass over the faces; the queues follow
         // windows: the queued faces wait for the band's end (they are
         // projected again from the corner table there); every wave is done
         // with this window's cache before the next one is projected.  The
         // window's flag goes to slot wslot, read after the barrier; the next
         // slot (last read two windows ago, before the previous barrier) is
         // cleared before it.
-        if (__ballot(fmask != 0ull) != 0ull && lane == 0) s_later[wslot] = 1;
+        if (any_later != 0ull && lane == 0) s_later[wslot] = 1;
         if (tid == 0) s_later[wslot == 2 ? 0 : wslot + 1] = 0;
         __syncthreads();
         if (wi < 64 && s_later[wslot] == 0) wmask &= ~(1ull << wi);
@@ -1188,7 +1313,8 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         }
         // the next band refills the tile; after the last one nothing reads
         // or writes it
-        if (b1 < ty1) __syncthreads();
+        if (more) __syncthreads();
+        first = false;
     }
 
     // carried pixels outside this iteration's union box stay as they are
@@ -1365,7 +1491,7 @@ __global__ __launch_bounds__(BT) void k_render_fitness_wrap(const QpsoSolveDev* 
         for (int v = tid; v < S.V_eff; v += BT) {
             int32_t X, Y;
             float Z;
-            dg |= vertex_fixed(pose, wx[v], wy[v], wz[v], cam, X, Y, Z) ? 1 : 0;
+            vertex_fixed(pose, wx[v], wy[v], wz[v], cam, X, Y, Z);
             xl = min(xl, X); xh = max(xh, X);
             yl = min(yl, Y); yh = max(yh, Y);
         }
@@ -1373,6 +1499,7 @@ __global__ __launch_bounds__(BT) void k_render_fitness_wrap(const QpsoSolveDev* 
         if (xl <= xh) {
             bx0 = wadd(xl, 15) >> 4; bx1 = wadd(xh, 15) >> 4;
             by0 = wadd(yl, 15) >> 4; by1 = wadd(yh, 15) >> 4;
+            dg = beyond_limit(xl, xh, yl, yh);
         }
         bx0 = wave_min(bx0); bx1 = wave_max(bx1);
         by0 = wave_min(by0); by1 = wave_max(by1);

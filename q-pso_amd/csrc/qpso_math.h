@@ -216,7 +216,6 @@ struct Face {
     int32_t X[3], Y[3];
     float Z[3];
     int32_t minx, maxx, miny, maxy;
-    bool degen;
 };
 
 QD void face_bbox(Face& fc) {
@@ -226,14 +225,19 @@ QD void face_bbox(Face& fc) {
     fc.maxy = wadd(max(max(fc.Y[0], fc.Y[1]), fc.Y[2]), 15) >> 4;
 }
 
-// Projected vertex in 28.4 fixed point; `degen` if outside the +-2^30 range.
-QD bool vertex_fixed(const float pose[7], float vx, float vy, float vz, const Cam& c,
+// Projected vertex in 28.4 fixed point.
+QD void vertex_fixed(const float pose[7], float vx, float vy, float vz, const Cam& c,
                      int32_t& X, int32_t& Y, float& Z) {
     float u, v;
     project(pose, vx, vy, vz, c, u, v, Z);
     X = rint_sat(16.0f * u);
     Y = rint_sat(16.0f * v);
-    return (X > QPSO_FXP_LIMIT) | (X < -QPSO_FXP_LIMIT) | (Y > QPSO_FXP_LIMIT) | (Y < -QPSO_FXP_LIMIT);
+}
+
+// Whether extremes of 28.4 coordinates leave the +-2^30 range (one of the
+// coordinates then does).
+QD int beyond_limit(int32_t xl, int32_t xh, int32_t yl, int32_t yh) {
+    return (xl < -QPSO_FXP_LIMIT) | (xh > QPSO_FXP_LIMIT) | (yl < -QPSO_FXP_LIMIT) | (yh > QPSO_FXP_LIMIT);
 }
 
 // Face f projected from the corner table (corner j of face f at
@@ -241,7 +245,6 @@ QD bool vertex_fixed(const float pose[7], float vx, float vy, float vz, const Ca
 QD void face_project(const float* __restrict__ corners, int f, const float pose[7], const Cam& c, Face& fc) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     const f4* __restrict__ cr = reinterpret_cast<const f4*>(corners) + 3 * (size_t)f;
-    fc.degen = false;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         const f4 w = cr[j];
@@ -250,8 +253,6 @@ QD void face_project(const float* __restrict__ corners, int f, const float pose[
         fc.X[j] = rint_sat(16.0f * u);
         fc.Y[j] = rint_sat(16.0f * v);
         fc.Z[j] = Z;
-        fc.degen |= (fc.X[j] > QPSO_FXP_LIMIT) | (fc.X[j] < -QPSO_FXP_LIMIT) |
-                    (fc.Y[j] > QPSO_FXP_LIMIT) | (fc.Y[j] < -QPSO_FXP_LIMIT);
     }
     face_bbox(fc);
 }
@@ -283,13 +284,14 @@ QD bool face_setup(const Face& fc, Setup& s) {
     const float inv = 1.0f * rcp((float)tri);
     s.FDX23 = wshl(DX23, 4); s.FDX31 = wshl(DX31, 4);
     s.FDY23 = wshl(DY23, 4); s.FDY31 = wshl(DY31, 4);
-    int32_t C2 = wsub(wmul(DY23, X2), wmul(DX23, Y2));
-    int32_t C3 = wsub(wmul(DY31, X3), wmul(DX31, Y3));
-    C2 = wadd(C2, (DY23 < 0 || (DY23 == 0 && DX23 > 0)) ? 1 : 0);
-    C3 = wadd(C3, (DY31 < 0 || (DY31 == 0 && DX31 > 0)) ? 1 : 0);
+    // the edge's value at its vertex is zero, so at the bbox origin (MINX,
+    // MINY) it is DY (X - MINX) - DX (Y - MINY) (equal modulo 2^32 to the
+    // reference's C + DX MINY - DY MINX), plus the top-left bias
     const int32_t MINY = wshl(fc.miny, 4), MINX = wshl(fc.minx, 4);
-    s.CY2 = wsub(wadd(C2, wmul(DX23, MINY)), wmul(DY23, MINX));
-    s.CY3 = wsub(wadd(C3, wmul(DX31, MINY)), wmul(DY31, MINX));
+    const int32_t C2 = wsub(wmul(DY23, wsub(X2, MINX)), wmul(DX23, wsub(Y2, MINY)));
+    const int32_t C3 = wsub(wmul(DY31, wsub(X3, MINX)), wmul(DX31, wsub(Y3, MINY)));
+    s.CY2 = wadd(C2, (DY23 < 0 || (DY23 == 0 && DX23 > 0)) ? 1 : 0);
+    s.CY3 = wadd(C3, (DY31 < 0 || (DY31 == 0 && DX31 > 0)) ? 1 : 0);
     s.z1 = fc.Z[0];
     s.z2 = (fc.Z[1] - fc.Z[0]) * inv;
     s.z3 = (fc.Z[2] - fc.Z[0]) * inv;

@@ -141,6 +141,13 @@ inline void build_mesh_tables(const float* A, uint32_t F, std::vector<float>& ve
     build_runs(tri, F, runs);
 }
 
+// The raster table as the device reads it: vertex indices modulo 65536.
+inline void build_index_table(const std::vector<QpsoFaceRef>& order, std::vector<QpsoFaceIdx>& out) {
+    out.resize(order.size());
+    for (size_t f = 0; f < order.size(); ++f)
+        out[f] = QpsoFaceIdx{(uint16_t)order[f].v0, (uint16_t)order[f].v1, (uint16_t)order[f].v2, 0};
+}
+
 // Corner j of face f (raster order): its mesh coordinates (x, y, z) and its
 // unique-vertex index as the bits of the fourth float.
 inline void build_corner_table(const float* soa, uint32_t F, const std::vector<QpsoFaceRef>& order,
