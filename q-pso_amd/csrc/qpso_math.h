@@ -36,6 +36,28 @@ QD int32_t rint_sat(float x) {
 
 QD float rcp(float x) { return 1.0f / x; }  // __frcp_rn
 
+// The same from one Newton step on v_rcp_f32, a third of the division's time.
+// e is the step's residual: wherever |e| < 2^-20 (every x with x and 1/x
+// normal; zero, denormal, huge, infinite and NaN x fail it) the result equals
+// 1.0f / x, compared for all 2^32 inputs on the device.
+QD float rcp_newton(float x, float& e) {
+    const float r0 = __builtin_amdgcn_rcpf(x);
+    const float r = __builtin_fmaf(__builtin_fmaf(-x, r0, 1.0f), r0, r0);
+    e = __builtin_fmaf(-x, r, 1.0f);
+    return r;
+}
+constexpr float kRcpOk = 0x1p-20f;
+QD float rcp_any(float x) {  // 1.0f / x for every x
+    float e;
+    float r = rcp_newton(x, e);
+    if (!(__builtin_fabsf(e) < kRcpOk)) r = 1.0f / x;
+    return r;
+}
+QD float rcp_normal(float x) {  // 1.0f / x where x and 1/x are normal
+    float e;
+    return rcp_newton(x, e);
+}
+
 // ---- sin / cos / acos (binary64 evaluation, one final rounding) ----------
 constexpr double kPio2Hi = 0x1.921fb54442d18p+0;
 constexpr double kPio2Lo = 0x1.1a62633145c07p-54;
@@ -190,25 +212,74 @@ struct Cam {
     double fx, fy, cx, cy;
 };
 
-QD void project(const float pose[7], float vx, float vy, float vz, const Cam& c,
-                float& u, float& v, float& Z) {
+// The rotation's 2 (q x v) takes its factor into the constants: doubling is
+// exact.
+QD void to_camera(const float pose[7], float vx, float vy, float vz, float& px, float& py, float& pz) {
     const float q0 = pose[3], q1 = pose[4], q2 = pose[5], q3 = pose[6];
-    const float t0 = 2.0f * __builtin_fmaf(q2, vz, -(q3 * vy));
-    const float t1 = 2.0f * -__builtin_fmaf(q1, vz, -(q3 * vx));
-    const float t2 = 2.0f * __builtin_fmaf(q1, vy, -(q2 * vx));
+    const float d1 = 2.0f * q1, d2 = 2.0f * q2, d3 = 2.0f * q3;
+    const float t0 = __builtin_fmaf(d2, vz, -(d3 * vy));
+    const float t1 = __builtin_fmaf(-d1, vz, d3 * vx);
+    const float t2 = __builtin_fmaf(d1, vy, -(d2 * vx));
     const float k0 = __builtin_fmaf(q2, t2, -(q3 * t1));
-    const float k1 = -__builtin_fmaf(q1, t2, -(q3 * t0));
+    const float k1 = __builtin_fmaf(-q1, t2, q3 * t0);
     const float k2 = __builtin_fmaf(q1, t1, -(q2 * t0));
-    float px = __builtin_fmaf(q0, t0, vx) + k0;
-    float py = __builtin_fmaf(q0, t1, vy) + k1;
-    float pz = __builtin_fmaf(q0, t2, vz) + k2;
+    px = __builtin_fmaf(q0, t0, vx) + k0;
+    py = __builtin_fmaf(q0, t1, vy) + k1;
+    pz = __builtin_fmaf(q0, t2, vz) + k2;
     px += pose[0];
     py += pose[1];
     pz += pose[2];
-    const float r = rcp(pz);
+}
+
+QD void project(const float pose[7], float vx, float vy, float vz, const Cam& c,
+                float& u, float& v, float& Z) {
+    float px, py, pz;
+    to_camera(pose, vx, vy, vz, px, py, pz);
+    const float r = rcp_any(pz);
     u = (float)__builtin_fma(c.fx, (double)(px * r), c.cx);
     v = (float)__builtin_fma(c.fy, (double)(py * r), c.cy);
     Z = 1000.0f * pz;
+}
+
+// The fast projection of a mesh's vertices: 28.4 coordinates before rounding
+// (the factor 16 taken into the camera, exact), valid where ok returns true
+// and both stay below kFastLimit in magnitude.  There adding kRound rounds
+// them half to even into the low mantissa bits, the 16-bit half directly.
+struct Cam16 {
+    double fx, fy, cx, cy;
+};
+constexpr float kFastLimit = 0x1p22f;
+constexpr float kRound = 0x1.8p23f;
+QD bool vertex_fast(const float pose[7], float vx, float vy, float vz, const Cam16& c, float& x, float& y, float& Z) {
+    float px, py, pz, e;
+    to_camera(pose, vx, vy, vz, px, py, pz);
+    const float r = rcp_newton(pz, e);
+    x = (float)__builtin_fma(c.fx, (double)(px * r), c.cx);
+    y = (float)__builtin_fma(c.fy, (double)(py * r), c.cy);
+    Z = 1000.0f * pz;
+    return __builtin_fabsf(e) < kRcpOk;
+}
+// minimum and maximum of numbers, one instruction (the library's forms first
+// quiet their operands; a NaN operand is passed over here too)
+QD float min_num(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+QD float max_num(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// X | Y << 16 of such coordinates
+QD uint32_t pack_fast(float x, float y) {
+    return __builtin_amdgcn_perm(__float_as_uint(y + kRound), __float_as_uint(x + kRound), 0x05040100u);
+}
+// whether the pose and the camera are numbers that vertex_fast takes
+QD bool fast_inputs(const float pose[7], const Cam& c) {
+    const double m = __builtin_fabs(c.fx) + __builtin_fabs(c.fy) + __builtin_fabs(c.cx) + __builtin_fabs(c.cy);
+    const float p = __builtin_fabsf(pose[0]) + __builtin_fabsf(pose[1]);
+    return m < 1e30 && p < 1e30f;
 }
 
 // Fixed-point face: 28.4 vertices and the integer bbox (main.h:1326-1353).
@@ -281,7 +352,7 @@ QD bool face_setup(const Face& fc, Setup& s) {
     const int32_t tri = wsub(wmul(DX12, DY31), wmul(DX31, DY12));
     if (tri <= 0) return false;
     if (fc.maxx - fc.minx <= 0 || fc.maxy - fc.miny <= 0) return false;
-    const float inv = 1.0f * rcp((float)tri);
+    const float inv = rcp_normal((float)tri);  // 1 <= tri < 2^31
     s.FDX23 = wshl(DX23, 4); s.FDX31 = wshl(DX31, 4);
     s.FDY23 = wshl(DY23, 4); s.FDY31 = wshl(DY31, 4);
     // the edge's value at its vertex is zero, so at the bbox origin (MINX,
