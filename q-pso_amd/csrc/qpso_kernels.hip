@@ -84,6 +84,21 @@ __device__ __forceinline__ unsigned long long wave_sum64(unsigned long long v) {
            ((unsigned long long)d << 48);
 }
 
+// The halving tree's last levels, v += v of the lane 32, 16, 8, 4, 2, 1 on;
+// the sum stands in lane 0.
+__device__ __forceinline__ float wave_halving(float v) {
+    const auto swapped = [](auto r) { return __builtin_bit_cast(float, (uint32_t)r[1]); };
+    uint32_t b = __builtin_bit_cast(uint32_t, v);
+    v = v + swapped(__builtin_amdgcn_permlane32_swap(b, b, false, false));
+    b = __builtin_bit_cast(uint32_t, v);
+    v = v + swapped(__builtin_amdgcn_permlane16_swap(b, b, false, false));
+    v = v + __int_as_float(dpp<0x108, 0xf>(0, __float_as_int(v)));  // row_shl:8
+    v = v + __int_as_float(dpp<0x104, 0xf>(0, __float_as_int(v)));
+    v = v + __int_as_float(dpp<0x102, 0xf>(0, __float_as_int(v)));
+    v = v + __int_as_float(dpp<0x101, 0xf>(0, __float_as_int(v)));
+    return v;
+}
+
 #define RT(S, p, s) (S).rand[(size_t)(p) + (size_t)(s) * (size_t)(S).N]
 
 // ------------------------------------------------------------------------
@@ -793,7 +808,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     int wslot = 0;
     bool first = true;
     for (int32_t b0 = ty0, b1; has_tile && b0 < ty1; b0 = b1) {
-        b1 = band_end(b0);  // band rows [b0, b1)
+        b1 = first && region + TW + 8 <= tcap ? ty1 : band_end(b0);  // band rows [b0, b1)
         const int32_t nb = b1 - b0;
         db0 = max(b0, dy0);
         const int32_t db1 = min(b1, dy1);
@@ -1134,7 +1149,8 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         // queued small faces: per-pixel depth over their D part, K lanes per
         // face (a power of two, as many as the threads allow, at most 64),
         // lane j of a face taking its pixels j, j + K, j + 2K, ...
-        const int nq = min(s_nq, kQCap);
+        const int nq = min(s_nq, kQCap), nqb = min(s_nqb, kBQCap);
+        if (nq + nqb > 0) {
         if (nq > 0) {
             const int share = BT / nq;
             const int K = share >= 64 ? 64 : share >= 1 ? 1 << (31 - __builtin_clz(share)) : 1;
@@ -1147,17 +1163,17 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                 raster_lanes(fc, su, max(fc.minx, dx0), min(fc.maxx, dx1), max(fc.miny, db0), min(fc.maxy, db1), j, K);
             }
         }
-        // queued big faces: one face per wave, taken in turn
-        const int nqb = min(s_nqb, kBQCap);
-        for (;;) {
-            int q = 0;
-            if ((tid & 63) == 0) q = atomicAdd(&s_take, 1);
-            q = __shfl(q, 0);
-            if (q >= nqb) break;
+        // queued big faces: one face per wave, the first by its number, the
+        // next ones taken in turn
+        for (int q = tid >> 6; q < nqb;) {
             raster_wave(q);
+            int t = 0;
+            if ((tid & 63) == 0) t = atomicAdd(&s_take, 1);
+            q = BT / 64 + __builtin_amdgcn_readfirstlane(t);
         }
         __syncthreads();
         if (tid == 0) { s_nq = 0; s_nqb = 0; s_take = 0; }
+        }
         }
 
         if (full) {  // D is the whole tile here
@@ -1445,12 +1461,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
 #pragma unroll
             for (int k = 0; k < s; ++k) r[k] = r[k] + r[k + s];
         }
-        float v = r[0];
-#pragma unroll
-        for (int stride = 32; stride >= 1; stride >>= 1) {
-            const float o = __shfl_down(v, stride);
-            v = v + o;
-        }
+        const float v = wave_halving(r[0]);
         if (tid == 0) {
             const uint32_t seg = s_cnt[0], tr = s_cnt[1], nr = s_cnt[2];
             const float inv_r = rcp((float)nr);
