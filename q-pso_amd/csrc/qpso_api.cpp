@@ -74,11 +74,17 @@ void free_mesh(Mesh& m) {
 
 struct ArenaLayout {
     size_t desc, obs, obs_rows, pos, vel, pbest, pbest_fit, fit, gbest, iter, flags, counters;
-    size_t stale0, stale1, cnt0, cnt1, fit_tr, gbest_tr, argmin_tr, frames, total;
+    size_t stale0, stale1, cnt0, cnt1, fit_tr, gbest_tr, argmin_tr, frames, pos1, fit1, gbest1, total;
 };
 
-// `wrap`: the reference-faithful off-frame mode's full per-particle buffers
-ArenaLayout layout(int N, int I, int rw, int rh, bool trace, bool wrap = false) {
+// Plain solves run with two buffers of pos, fit and gbest up to this many
+// particles (each workgroup of a PSO step reads every particle's fitness, so
+// the sum grows with the square).
+constexpr int kMaxTwoBuffers = 4096;
+
+// `wrap`: the reference-faithful off-frame mode's full per-particle buffers;
+// `two`: the second buffers of pos, fit and gbest
+ArenaLayout layout(int N, int I, int rw, int rh, bool trace, bool wrap = false, bool two = false) {
     ArenaLayout L{};
     size_t o = 0;
     auto take = [&](size_t bytes) { size_t r = o; o = align_up(o + bytes, 256); return r; };
@@ -104,6 +110,11 @@ ArenaLayout layout(int N, int I, int rw, int rh, bool trace, bool wrap = false) 
         L.argmin_tr = take(sizeof(int32_t) * (size_t)I);
     }
     if (wrap) L.frames = take(sizeof(int32_t) * (size_t)N * kFrame);
+    if (two) {
+        L.pos1 = take(sizeof(float) * 7 * N);
+        L.fit1 = take(sizeof(float) * N);
+        L.gbest1 = take(sizeof(float) * 8);
+    }
     L.total = o;
     return L;
 }
@@ -160,6 +171,11 @@ void fill_desc(QpsoSolveDev& h, const Mesh& m, const qpso_cluster* cl, const qps
     if (p->offframe) {
         h.wrap = 1;
         h.frames = reinterpret_cast<int32_t*>(A + L.frames);
+    }
+    if (L.pos1) {
+        h.pos1 = reinterpret_cast<float*>(A + L.pos1);
+        h.fit1 = reinterpret_cast<float*>(A + L.fit1);
+        h.gbest1 = reinterpret_cast<float*>(A + L.gbest1);
     }
 }
 
@@ -393,10 +409,31 @@ bool any_needs_windows(qpso_solve* const* solves, int n, int cfg) {
     return false;
 }
 
+// One solve with two buffers: InitQPSO and its iterations.  With at most as
+// many particles as CUs the PSO step runs inside the next render launch: it
+// takes a workgroup 3.3 us, a launch of its own 6 (10k faces, 256 particles:
+// 7,900 -> 7,610 us).  With more, every round of workgroups would pay it
+// (1,024 particles: 3,600 -> 3,700 us).
+hipError_t launch_two_buffers(const QpsoSolveDev& h, int cfg, int n_cu, const QpsoSolveDev* d_desc, hipStream_t st) {
+    const int win = qpso_launch::rf_needs_windows(cfg, h.V_eff) ? 1 : 0;
+    const bool inside = h.N <= n_cu;
+    hipError_t e = qpso_launch::init(d_desc, 1, st, nullptr, nullptr, true);
+    for (int it = 0; it < h.I && e == hipSuccess; ++it) {
+        e = qpso_launch::render_fitness(cfg, win, d_desc, nullptr, h.N, st, nullptr, nullptr,
+                                        inside ? it : it | QPSO_STEP_APART);
+        if (e == hipSuccess && (!inside || it == h.I - 1)) e = qpso_launch::pso_step_two(d_desc, h.N, it, st);
+    }
+    return e;
+}
+
 // Launch the whole iteration loop of one solve (plain form).
 int launch_solve(qpso_solve* s, hipStream_t st) {
     qpso_ctx* ctx = s->ctx;
     if (s->h.wrap) HIP_TRY(ctx, qpso_launch::fill_frames(s->h.frames, (size_t)s->h.N * kFrame, st));
+    if (s->h.pos1) {
+        HIP_TRY(ctx, launch_two_buffers(s->h, s->rf_cfg, ctx->n_cu, s->d_desc, st));
+        return QPSO_OK;
+    }
     HIP_TRY(ctx, qpso_launch::init(s->d_desc, 1, st));
     for (int it = 0; it < s->h.I; ++it) {
         HIP_TRY(ctx, launch_rf(s, s->rf_cfg, s->d_desc, nullptr, s->h.N, st));
@@ -583,8 +620,11 @@ uint64_t qpso_solve_bytes(const qpso_params* p, const int32_t rect[4]) {
     return layout(p->n_particles, p->n_iters, rw, rh, false, p->offframe != 0).total;
 }
 
-int qpso_solve_create(qpso_ctx* ctx, uint32_t mesh_id, const qpso_cluster* cl, const qpso_params* p,
-                      int with_trace, qpso_solve** out) {
+namespace {
+
+// `plain`: the solve may run on its own (a server's never does)
+int create_solve(qpso_ctx* ctx, uint32_t mesh_id, const qpso_cluster* cl, const qpso_params* p, int with_trace,
+                 bool plain, qpso_solve** out) {
     if (!ctx || !out) return QPSO_E_INVAL;
     *out = nullptr;
     if (int v = validate(cl, p)) return set_err(ctx, v, "invalid cluster or parameters");
@@ -601,7 +641,7 @@ int qpso_solve_create(qpso_ctx* ctx, uint32_t mesh_id, const qpso_cluster* cl, c
     s->params = *p;
     s->mesh_id = mesh_id;
     std::memcpy(s->rect, cl->rect, sizeof(s->rect));
-    s->L = layout(N, I, rw, rh, s->trace, p->offframe != 0);
+    s->L = layout(N, I, rw, rh, s->trace, p->offframe != 0, plain && !p->offframe && N <= kMaxTwoBuffers);
     if (alloc_arena(ctx, s->L.total, &s->arena) != hipSuccess)
         return set_err(ctx, QPSO_E_NOMEM, "solve arena allocation failed");
     float* rand = nullptr;
@@ -639,8 +679,6 @@ int qpso_solve_create(qpso_ctx* ctx, uint32_t mesh_id, const qpso_cluster* cl, c
     return QPSO_OK;
 }
 
-namespace {
-
 // Destroy a solve whose work all lies on stream `st`; its arena is released
 // in that stream's order.
 void solve_release(qpso_solve* s, hipStream_t st) {
@@ -660,6 +698,11 @@ void solve_release(qpso_solve* s, hipStream_t st) {
 }
 
 }  // namespace
+
+int qpso_solve_create(qpso_ctx* ctx, uint32_t mesh_id, const qpso_cluster* cl, const qpso_params* p,
+                      int with_trace, qpso_solve** out) {
+    return create_solve(ctx, mesh_id, cl, p, with_trace, true, out);
+}
 
 int qpso_solve_destroy(qpso_solve* s) {
     if (!s) return QPSO_E_INVAL;
@@ -808,9 +851,11 @@ int qpso_estimate_pose_noalloc(qpso_ctx* ctx, uint32_t mesh_id, const qpso_clust
     const int N = p->n_particles, I = p->n_iters, S = qpso_host::rand_stride(I);
     const int rw = cl->rect[2] - cl->rect[0], rh = cl->rect[3] - cl->rect[1];
     // the arena as a solve's, then its random table
-    const ArenaLayout L = layout(N, I, rw, rh, false);
-    const size_t rand_off = align_up(L.total, 256);
     const size_t n_rand = (size_t)S * N;
+    ArenaLayout L = layout(N, I, rw, rh, false, false, N <= kMaxTwoBuffers);
+    // the second buffers only where everything fits with them
+    if (align_up(L.total, 256) + sizeof(float) * n_rand > QPSO_NOALLOC_SCRATCH_BYTES) L = layout(N, I, rw, rh, false);
+    const size_t rand_off = align_up(L.total, 256);
     if (rand_off + sizeof(float) * n_rand > QPSO_NOALLOC_SCRATCH_BYTES)
         return set_err(ctx, QPSO_E_NOMEM,
                        "solve needs " + std::to_string((rand_off + sizeof(float) * n_rand) >> 10) +
@@ -842,9 +887,10 @@ int qpso_estimate_pose_noalloc(qpso_ctx* ctx, uint32_t mesh_id, const qpso_clust
     HIP_TRY(ctx, qpso_launch::obs_rows(reinterpret_cast<const uint16_t*>(A + L.obs),
                                        reinterpret_cast<uint16_t*>(A + L.obs_rows), rw, rh, st));
     // InitQPSO clears the iteration, flags, counters and carried-pixel counts
-    HIP_TRY(ctx, qpso_launch::init(d_desc, 1, st));
+    if (h.pos1) HIP_TRY(ctx, launch_two_buffers(h, ctx->rf_cfg, ctx->n_cu, d_desc, st));
+    else HIP_TRY(ctx, qpso_launch::init(d_desc, 1, st));
     const bool win = qpso_launch::rf_needs_windows(ctx->rf_cfg, h.V_eff);
-    for (int it = 0; it < I; ++it) {
+    for (int it = 0; it < I && !h.pos1; ++it) {
         HIP_TRY(ctx, qpso_launch::render_fitness(ctx->rf_cfg, win, d_desc, nullptr, N, st));
         HIP_TRY(ctx, qpso_launch::pso_step(d_desc, 1, st));
     }
@@ -1217,7 +1263,7 @@ struct HipDev {
 
     int create(Job& j, qpso_solve*& s) {
         j.cl.depth = j.depth.data();
-        const int rc = qpso_solve_create(ctx, j.mesh_id, &j.cl, &j.p, 0, &s);
+        const int rc = create_solve(ctx, j.mesh_id, &j.cl, &j.p, 0, false, &s);
         if (rc) return rc;
         s->rf_cfg = rf_cfg;  // the server's tuning, not the context's current one
         s->h.big_face = big_face;

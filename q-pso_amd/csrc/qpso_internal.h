@@ -28,6 +28,9 @@
 // device scratch of the allocation-free entry point (qpso_estimate_pose_noalloc)
 #define QPSO_NOALLOC_SCRATCH_BYTES QPSO_NOALLOC_BYTES
 
+// render_fitness iteration argument: the PSO step has a launch of its own
+#define QPSO_STEP_APART (1 << 30)
+
 struct QpsoStale {  // one carried-over depth-buffer pixel
     int32_t pos;    // (y << 16) | x
     int32_t val;
@@ -87,6 +90,10 @@ struct QpsoSolveDev {
     float* fit;             // [N]
     float* gbest;           // [8]: pose + fit
     int32_t* iter;          // [1]
+    // second buffers of a solve that may run with two (nullable)
+    float* pos1;            // [7][N]
+    float* fit1;            // [N]
+    float* gbest1;          // [8]
     QpsoStale* stale[2];    // [N][stale_cap] each
     int32_t* stale_cnt[2];  // [N] each
     int32_t stale_cap;

@@ -101,12 +101,23 @@ __device__ __forceinline__ float wave_halving(float v) {
 
 #define RT(S, p, s) (S).rand[(size_t)(p) + (size_t)(s) * (size_t)(S).N]
 
+// A solve run with two buffers of pos, fit and gbest: iteration it's are the
+// second ones (pos1, ...) where this is true.  The step after iteration it
+// reads them and writes the others, so that workgroups still reading never
+// meet a write; the last step leaves the results in the first ones.
+__device__ __forceinline__ bool step_buffer(const QpsoSolveDev& S, int it) { return ((it + S.I) & 1) != 0; }
+
 // ------------------------------------------------------------------------
 // InitQPSO (main.cu:72-198) + QuatKinematicsPSOStateVectWithInit (main.h:267-307)
 // ------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_init(const QpsoSolveDev* __restrict__ solves) {
+// two_buffers: a solve run with `it` (see k_render_fitness) starts in the
+// buffers of iteration 0.
+__global__ __launch_bounds__(256) void k_init(const QpsoSolveDev* __restrict__ solves, int two_buffers) {
     const QpsoSolveDev& S = solves[blockIdx.x];
     const int N = S.N;
+    const bool second = two_buffers && step_buffer(S, 0);
+    float* const pos = second ? S.pos1 : S.pos;
+    float* const gbest = second ? S.gbest1 : S.gbest;
     for (int p = threadIdx.x; p < N; p += blockDim.x) {
         float P[7], V[7];
         int s = 0;
@@ -128,7 +139,7 @@ __global__ __launch_bounds__(256) void k_init(const QpsoSolveDev* __restrict__ s
         for (int d = 0; d < 3; ++d) { V[4 + d] = __builtin_fmaf(20.0f, RT(S, p, s), -10.0f); ++s; }
 #pragma unroll
         for (int d = 0; d < 7; ++d) {
-            S.pos[d * N + p] = P[d];
+            pos[d * N + p] = P[d];
             S.vel[d * N + p] = V[d];
             S.pbest[d * N + p] = P[d];
         }
@@ -138,8 +149,8 @@ __global__ __launch_bounds__(256) void k_init(const QpsoSolveDev* __restrict__ s
     }
     if (threadIdx.x == 0) {
 #pragma unroll
-        for (int d = 0; d < 7; ++d) S.gbest[d] = 0.0f;
-        S.gbest[7] = QPSO_BEST_FIT_INIT;
+        for (int d = 0; d < 7; ++d) gbest[d] = 0.0f;
+        gbest[7] = QPSO_BEST_FIT_INIT;
         *S.iter = 0;
         *S.flags = 0;
         S.counters[0] = 0;
@@ -170,6 +181,171 @@ struct Visits {
         return ((__mul24(k, W) < T && !short_row(k)) ? 1 : 0) + ((__mul24(k + 1, W) < T && short_row(k + 1)) ? 1 : 0);
     }
 };
+
+// ------------------------------------------------------------------------
+// one particle's update (main.cu:786-1060)
+// ------------------------------------------------------------------------
+// The state one particle update reads, held in registers.
+struct Particle {
+    float P[7], V[7], B[7];  // pos, vel, pbest
+    float R[12];             // the iteration's random numbers, in order of use
+    float fit, pbest_fit;
+};
+
+// second: from the second buffers
+__device__ __forceinline__ void load_particle(const QpsoSolveDev& S, int p, int iter, bool second, Particle& q) {
+    const int N = S.N;
+    const QG float* __restrict__ pos = (const QG float*)(second ? S.pos1 : S.pos);
+    const QG float* __restrict__ vel = (const QG float*)S.vel;
+    const QG float* __restrict__ pb = (const QG float*)S.pbest;
+#pragma unroll
+    for (int d = 0; d < 7; ++d) {
+        q.P[d] = pos[d * N + p];
+        q.V[d] = vel[d * N + p];
+        q.B[d] = pb[d * N + p];
+    }
+    q.fit = ((const QG float*)(second ? S.fit1 : S.fit))[p];
+    q.pbest_fit = ((const QG float*)S.pbest_fit)[p];
+    // d_randIdx: 12 at init + 12 per iteration; a finished solve (iter = I,
+    // values unused) reads the table's last rows instead of past its end
+    const int s0 = min(12 + 12 * iter, S.S - 12);
+    const QG float* __restrict__ rt = (const QG float*)S.rand;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) q.R[k] = rt[(size_t)p + (size_t)(s0 + k) * (size_t)N];
+}
+
+// The angular velocity that turns orientation P into T (main.cu:921-1031):
+// the log of T (x) conj(P) in the upper half, zero for a turn of no size.
+__device__ __forceinline__ void rotation_to(const float* T, const float* P, float o[3]) {
+    float qt[4];
+    qprod_conj(T, P, qt);
+    top_half(qt);
+    float n2 = __builtin_fmaf(qt[1], qt[1], qt[2] * qt[2]);
+    n2 = __builtin_fmaf(qt[3], qt[3], n2);
+    const float n = __builtin_sqrtf(n2);
+    if (n > 1.0e-7f) {
+        const float sc = (2.0f * acosf_q(qt[0])) * rcp(n);
+        o[0] = qt[1] * sc; o[1] = qt[2] * sc; o[2] = qt[3] * sc;
+    }
+}
+
+// UpdateParticlesEquationKernel (main.cu:858-1060) for one particle, gb = gbest.
+// PAIR: the particle's state is the same in every lane of the wave; even
+// lanes work out the turn to pbest, odd ones the turn to gbest.
+template <bool PAIR>
+__device__ __forceinline__ void step_particle(const QpsoSolveDev& S, Particle& q, const float* gb) {
+    float* P = q.P;
+    float* V = q.V;
+    const float* B = q.B;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const float r1 = S.c1 * q.R[2 * d];
+        const float r2 = S.c2 * q.R[2 * d + 1];
+        const float iV = (float)(S.w * (double)V[d]);
+        float v = __builtin_fmaf(r1, B[d] - P[d], iV);
+        v = __builtin_fmaf(r2, gb[d] - P[d], v);
+        V[d] = v;
+        P[d] += v;
+        if (P[d] < S.x_lo[d]) { P[d] = S.x_lo[d]; V[d] = 0.0f; }
+        else if (P[d] > S.x_hi[d]) { P[d] = S.x_hi[d]; V[d] = 0.0f; }
+    }
+    float wc[3] = {0.0f, 0.0f, 0.0f}, ws[3] = {0.0f, 0.0f, 0.0f};
+    if (PAIR) {
+        const bool odd = threadIdx.x & 1;
+        float T[4], o[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) T[i] = odd ? gb[3 + i] : B[3 + i];
+        rotation_to(T, &P[3], o);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            wc[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(o[i]), 0));
+            ws[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(o[i]), 1));
+        }
+    } else {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+        rotation_to(k == 0 ? &B[3] : &gb[3], &P[3], k == 0 ? wc : ws);
+    }
+    V[3] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const float r1 = S.c1 * q.R[6 + 2 * i];
+        const float r2 = S.c2 * q.R[7 + 2 * i];
+        const float iW = (float)(S.w * (double)V[4 + i]);
+        const float v = __builtin_fmaf(r1, wc[i], iW);
+        V[4 + i] = __builtin_fmaf(r2, ws[i], v);
+    }
+    float qq[4] = {P[3], P[4], P[5], P[6]};
+    kinematics_from(qq, &P[3], &V[4]);
+}
+
+// The PSO step of iteration it - 1 for particle p, by wave 0 of its workgroup
+// at the start of iteration it's render launch: the argmin over the
+// iteration's fitness (first index on ties, NaN never chosen), gbest, the
+// personal best, the update.  Every workgroup of the solve finds the same
+// gbest; workgroup 0 stores it.  A launch of k_pso_step of its own took 4.9 us
+// an iteration and its gap 1.3 us; this takes 3.3.
+__device__ __forceinline__ void step_in_launch(const QpsoSolveDev& S, int p, int it, float* s_pose) {
+    const int lane = threadIdx.x, N = S.N, prev = it - 1;
+    const bool odd = step_buffer(S, prev);
+    const QG float* __restrict__ fit = (const QG float*)(odd ? S.fit1 : S.fit);
+    const QG float* __restrict__ pos = (const QG float*)(odd ? S.pos1 : S.pos);
+    const QG float* __restrict__ gold = (const QG float*)(odd ? S.gbest1 : S.gbest);
+    Particle q;
+    load_particle(S, p, prev, odd, q);
+    float g[8];
+#pragma unroll
+    for (int d = 0; d < 8; ++d) g[d] = gold[d];
+    float bv = __builtin_inff();
+    int bi = INT32_MAX;
+    for (int k = lane; k < N; k += 64) {
+        const float v = fit[k];
+        if (v == v && (bi == INT32_MAX || v < bv)) { bv = v; bi = k; }
+    }
+    const float m = __int_as_float(wave_reduce(__float_as_int(bv), __float_as_int(__builtin_inff()), [](int a, int b) {
+        return __float_as_int(min_num(__int_as_float(a), __int_as_float(b)));
+    }));
+    bi = wave_min(bi != INT32_MAX && bv == m ? bi : INT32_MAX);
+    const bool gnew = bi != INT32_MAX && m < g[7];
+    if (gnew) {
+#pragma unroll
+        for (int d = 0; d < 7; ++d) g[d] = pos[d * N + bi];
+        g[7] = m;
+    }
+    if (p == 0 && lane == 0) {
+        float* const gout = odd ? S.gbest : S.gbest1;
+#pragma unroll
+        for (int d = 0; d < 8; ++d) gout[d] = g[d];
+        if (S.gbest_trace) {
+#pragma unroll
+            for (int d = 0; d < 8; ++d) S.gbest_trace[(size_t)prev * 8 + d] = g[d];
+        }
+        if (S.argmin_trace) S.argmin_trace[prev] = bi == INT32_MAX ? 0 : bi;
+    }
+    const bool pnew = q.fit < q.pbest_fit;
+    if (pnew) {
+#pragma unroll
+        for (int d = 0; d < 7; ++d) q.B[d] = q.P[d];
+    }
+    if (lane == 0) {
+        if (S.fit_trace) S.fit_trace[(size_t)prev * N + p] = q.fit;
+        if (pnew) {
+            S.pbest_fit[p] = q.fit;
+#pragma unroll
+            for (int d = 0; d < 7; ++d) S.pbest[d * N + p] = q.B[d];
+        }
+    }
+    step_particle<true>(S, q, g);
+    if (lane == 0) {
+        float* const pout = odd ? S.pos : S.pos1;
+#pragma unroll
+        for (int d = 0; d < 7; ++d) {
+            pout[d * N + p] = q.P[d];
+            S.vel[d * N + p] = q.V[d];
+            s_pose[d] = q.P[d];
+        }
+    }
+}
 
 // Waves per SIMD when as many workgroups as the LDS allows share a CU (160
 // KiB of LDS, 4 SIMDs): the register budget both bodies of a windowed
@@ -231,13 +407,14 @@ struct RfLds {
     int32_t s_later[3];  // a face of the window reaches later bands (slot: windows drawn mod 3)
     uint32_t s_cnt[3];   // seg, tr, n_rendered
     unsigned long long s_px[2];
+    float s_pose[7];     // the particle's pose, from the PSO step inside the launch
 };
 
 // WIN: the body that can draw a mesh window by window (larger than the vertex
 // cache); the other one keeps the cached path free of it.
 template <int BT, int CAP, int MODE>
 __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves, const QpsoItem* __restrict__ items,
-                                        RfLds<CAP>& sh) {
+                                        RfLds<CAP>& sh, int it) {
     constexpr bool WIN = MODE >= 1;     // meshes beyond the vertex cache, window by window
     constexpr bool FRAMES = MODE == 2;  // and the frame dump (stage calls)
     constexpr int PR = 1024 / BT;  // pairs of fitness slots per thread
@@ -264,11 +441,16 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     // cache).  Then the carried pixels (at most QPSO_STALE_CAP, kSPT per
     // thread, kept in registers for the whole pass).  All are in bounds
     // whatever the iteration, so they load before the finished-solve test.
+    // With it >= 0 (two buffers) the iteration is it; with the PSO step inside
+    // this launch the pose comes from wave 0's step through LDS.
     const int N = S.N;
-    const int iter_v = ((const QG int32_t*)S.iter)[0];
+    const bool inside = it > 0 && !(it & QPSO_STEP_APART);
+    const bool second = it >= 0 && step_buffer(S, it & ~QPSO_STEP_APART);
+    const int iter_v = it >= 0 ? it & ~QPSO_STEP_APART : ((const QG int32_t*)S.iter)[0];
     float pose[7];
 #pragma unroll
-    for (int d = 0; d < 7; ++d) pose[d] = ((const QG float*)S.pos)[d * N + p];
+    for (int d = 0; d < 7; ++d) pose[d] = ((const QG float*)(second ? S.pos1 : S.pos))[d * N + p];
+    float* const fit_out = second ? S.fit1 : S.fit;
     const int n_old0 = ((const QG int32_t*)S.stale_cnt[0])[p];
     const int n_old1 = ((const QG int32_t*)S.stale_cnt[1])[p];
     constexpr int kWin = CAP / 6;  // vertex cache capacity
@@ -301,7 +483,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     // each instantiation only for the meshes and outputs it handles
     if ((!WIN && Ve > kWin) || (!FRAMES && S.dbg_frames)) {
         if (tid == 0) {
-            S.fit[p] = __builtin_nanf("");
+            fit_out[p] = __builtin_nanf("");
             atomicOr(S.flags, QPSO_FLAG_LAUNCH);
         }
         return;
@@ -324,6 +506,10 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         s_px[0] = s_px[1] = 0;
     }
     __syncthreads();
+    if (inside) {
+#pragma unroll
+        for (int d = 0; d < 7; ++d) pose[d] = sh.s_pose[d];
+    }
 
     // The projected unique vertices stay in LDS, one word each: X and Y in 28.4
     // as 16-bit halves, which the cull reads with packed 16-bit instructions.
@@ -473,7 +659,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
 
     if (degen) {  // guard G: NaN fitness, buffer reset
         if (tid == 0) {
-            S.fit[p] = __builtin_nanf("");
+            fit_out[p] = __builtin_nanf("");
             S.stale_cnt[par ^ 1][p] = 0;
             atomicAdd(&S.counters[2], 1ull);
         }
@@ -1468,7 +1654,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             const float ratio = (float)seg * rcp((float)S.num_points);
             const float ratioT = (float)tr * inv_r;
             const float zerr = v * inv_r;
-            S.fit[p] = (float)__builtin_fma((double)(ratio + ratioT), 0.05, (double)zerr);
+            fit_out[p] = (float)__builtin_fma((double)(ratio + ratioT), 0.05, (double)zerr);
             const int ns = s_nstale;
             S.stale_cnt[par ^ 1][p] = ns < cap ? ns : cap;
             atomicAdd(&S.counters[0], s_px[0]);
@@ -1482,16 +1668,21 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
 // cached meshes take the windowless body, which is faster for them.
 template <int BT, int CAP, int MODE>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(rf_waves_per_simd(BT, CAP))))
-void k_render_fitness(const QpsoSolveDev* __restrict__ solves, const QpsoItem* __restrict__ items) {
+void k_render_fitness(const QpsoSolveDev* __restrict__ solves, const QpsoItem* __restrict__ items, int it) {
     __shared__ RfLds<CAP> sh;
+    // plain solves: iteration it - 1's PSO step first (its barrier is the
+    // body's first); a scalar branch, since under a vector one the compiler
+    // spills the body's registers
+    if (it > 0 && !(it & QPSO_STEP_APART) && __builtin_amdgcn_readfirstlane(threadIdx.x) < 64)
+        step_in_launch(solves[0], (int)blockIdx.x, it, sh.s_pose);
     if (MODE == 1) {
         const QpsoItem item = items ? items[blockIdx.x] : QpsoItem{0, (int32_t)blockIdx.x};
         if (solves[item.solve].V_eff <= CAP / 6) {
-            rf_body<BT, CAP, 0>(solves, items, sh);
+            rf_body<BT, CAP, 0>(solves, items, sh, it);
             return;
         }
     }
-    rf_body<BT, CAP, MODE>(solves, items, sh);
+    rf_body<BT, CAP, MODE>(solves, items, sh, it);
 }
 
 // ------------------------------------------------------------------------
@@ -1755,81 +1946,8 @@ __device__ __forceinline__ bool better(float av, int ai, float bv, int bi) {
     return av < bv || (av == bv && ai < bi);
 }
 
-// The state one particle update reads, held in registers.
-struct Particle {
-    float P[7], V[7], B[7];  // pos, vel, pbest
-    float R[12];             // the iteration's random numbers, in order of use
-    float fit, pbest_fit;
-};
-
-__device__ __forceinline__ void load_particle(const QpsoSolveDev& S, int p, int iter, Particle& q) {
-    const int N = S.N;
-    const QG float* __restrict__ pos = (const QG float*)S.pos;
-    const QG float* __restrict__ vel = (const QG float*)S.vel;
-    const QG float* __restrict__ pb = (const QG float*)S.pbest;
-#pragma unroll
-    for (int d = 0; d < 7; ++d) {
-        q.P[d] = pos[d * N + p];
-        q.V[d] = vel[d * N + p];
-        q.B[d] = pb[d * N + p];
-    }
-    q.fit = ((const QG float*)S.fit)[p];
-    q.pbest_fit = ((const QG float*)S.pbest_fit)[p];
-    // d_randIdx: 12 at init + 12 per iteration; a finished solve (iter = I,
-    // values unused) reads the table's last rows instead of past its end
-    const int s0 = min(12 + 12 * iter, S.S - 12);
-    const QG float* __restrict__ rt = (const QG float*)S.rand;
-#pragma unroll
-    for (int k = 0; k < 12; ++k) q.R[k] = rt[(size_t)p + (size_t)(s0 + k) * (size_t)N];
-}
-
-// UpdateParticlesEquationKernel (main.cu:858-1060) for one particle, gb = gbest
-__device__ void step_particle(const QpsoSolveDev& S, Particle& q, const float* gb) {
-    float* P = q.P;
-    float* V = q.V;
-    const float* B = q.B;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const float r1 = S.c1 * q.R[2 * d];
-        const float r2 = S.c2 * q.R[2 * d + 1];
-        const float iV = (float)(S.w * (double)V[d]);
-        float v = __builtin_fmaf(r1, B[d] - P[d], iV);
-        v = __builtin_fmaf(r2, gb[d] - P[d], v);
-        V[d] = v;
-        P[d] += v;
-        if (P[d] < S.x_lo[d]) { P[d] = S.x_lo[d]; V[d] = 0.0f; }
-        else if (P[d] > S.x_hi[d]) { P[d] = S.x_hi[d]; V[d] = 0.0f; }
-    }
-    float wc[3] = {0.0f, 0.0f, 0.0f}, ws[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        float qt[4];
-        qprod_conj(k == 0 ? &B[3] : &gb[3], &P[3], qt);
-        top_half(qt);
-        float n2 = __builtin_fmaf(qt[1], qt[1], qt[2] * qt[2]);
-        n2 = __builtin_fmaf(qt[3], qt[3], n2);
-        const float n = __builtin_sqrtf(n2);
-        if (n > 1.0e-7f) {
-            const float sc = (2.0f * acosf_q(qt[0])) * rcp(n);
-            float* o = k == 0 ? wc : ws;
-            o[0] = qt[1] * sc; o[1] = qt[2] * sc; o[2] = qt[3] * sc;
-        }
-    }
-    V[3] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const float r1 = S.c1 * q.R[6 + 2 * i];
-        const float r2 = S.c2 * q.R[7 + 2 * i];
-        const float iW = (float)(S.w * (double)V[4 + i]);
-        const float v = __builtin_fmaf(r1, wc[i], iW);
-        V[4 + i] = __builtin_fmaf(r2, ws[i], v);
-    }
-    float qq[4] = {P[3], P[4], P[5], P[6]};
-    kinematics_from(qq, &P[3], &V[4]);
-}
-
 // personal best (strict <, main.cu:786-811), then the update; stores the particle
-__device__ __forceinline__ void finish_particle(const QpsoSolveDev& S, int p, Particle& q, const float* gb) {
+__device__ __forceinline__ void finish_particle(const QpsoSolveDev& S, int p, Particle& q, const float* gb, float* pos) {
     const int N = S.N;
     if (q.fit < q.pbest_fit) {
         S.pbest_fit[p] = q.fit;
@@ -1839,10 +1957,10 @@ __device__ __forceinline__ void finish_particle(const QpsoSolveDev& S, int p, Pa
             S.pbest[d * N + p] = q.P[d];
         }
     }
-    step_particle(S, q, gb);
+    step_particle<false>(S, q, gb);
 #pragma unroll
     for (int d = 0; d < 7; ++d) {
-        S.pos[d * N + p] = q.P[d];
+        pos[d * N + p] = q.P[d];
         S.vel[d * N + p] = q.V[d];
     }
 }
@@ -1851,35 +1969,41 @@ __device__ __forceinline__ void finish_particle(const QpsoSolveDev& S, int p, Pa
 // the step waits on one round of loads (more when N > BT).  Every thread
 // finishes the argmin from the per-wave winners, and the owner of the winner
 // hands its pose to the others through LDS.
+//   it >= 0: one solve with two buffers, one workgroup per BT particles, each
+// finding the same argmin over all (1,024 particles in one workgroup took
+// 13.6 us, 2,048 took 25; one particle a thread takes 5).
 template <int BT>
-__global__ __launch_bounds__(BT) void k_pso_step(const QpsoSolveDev* __restrict__ solves) {
+__global__ __launch_bounds__(BT) void k_pso_step(const QpsoSolveDev* __restrict__ solves, int it) {
     constexpr int kWaves = BT / 64;
     __shared__ float s_v[kWaves];
     __shared__ int s_i[kWaves];
     __shared__ float s_pos[7];
-    const QpsoSolveDev& S = solves[blockIdx.x];
+    const bool two = it >= 0;
+    const QpsoSolveDev& S = solves[two ? 0 : blockIdx.x];
     const int tid = threadIdx.x;
     const int N = S.N;
-    const int iter = __builtin_amdgcn_readfirstlane(((const QG int32_t*)S.iter)[0]);
+    const int iter = two ? it : __builtin_amdgcn_readfirstlane(((const QG int32_t*)S.iter)[0]);
+    const bool second = two && step_buffer(S, it);
+    const float* const fit = second ? S.fit1 : S.fit;
+    float* const pos_in = second ? S.pos1 : S.pos;
+    float* const pos_out = two && !second ? S.pos1 : S.pos;
+    float* const gb_out = two && !second ? S.gbest1 : S.gbest;
+    const int p0 = (two ? (int)blockIdx.x * BT : 0) + tid;
     Particle q0;
-    if (tid < N) load_particle(S, tid, iter, q0);
+    if (p0 < N) load_particle(S, p0, iter, second, q0);
     float g[8];
 #pragma unroll
-    for (int d = 0; d < 8; ++d) g[d] = ((const QG float*)S.gbest)[d];
+    for (int d = 0; d < 8; ++d) g[d] = ((const QG float*)(second ? S.gbest1 : S.gbest))[d];
     if (iter >= S.I) return;
 
     // argmin, first index on ties, NaN never chosen (thrust::min_element,
     // main.cu:1691-1698)
     float bv = 0.0f;
     int bi = INT32_MAX;
-    if (tid < N) {
-        if (q0.fit == q0.fit) { bv = q0.fit; bi = tid; }
-        if (S.fit_trace) S.fit_trace[(size_t)iter * N + tid] = q0.fit;
-    }
-    for (int p = tid + BT; p < N; p += BT) {
-        const float v = S.fit[p];
+    for (int p = tid; p < N; p += BT) {
+        const float v = p == p0 ? q0.fit : fit[p];
         if (v == v && better(v, p, bv, bi)) { bv = v; bi = p; }
-        if (S.fit_trace) S.fit_trace[(size_t)iter * N + p] = v;
+        if (S.fit_trace && (!two || p == p0)) S.fit_trace[(size_t)iter * N + p] = v;
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -1900,19 +2024,24 @@ __global__ __launch_bounds__(BT) void k_pso_step(const QpsoSolveDev* __restrict_
     // NaN, when no comparison succeeds
     const bool gnew = bi != INT32_MAX && bv < g[7];
     if (gnew) {
-        if (tid == best % BT) {
+        if (two) {  // read by every thread; nothing writes it in this launch
 #pragma unroll
-            for (int d = 0; d < 7; ++d) s_pos[d] = best < BT ? q0.P[d] : S.pos[d * N + best];
+            for (int d = 0; d < 7; ++d) g[d] = pos_in[d * N + best];
+        } else {
+            if (tid == best % BT) {
+#pragma unroll
+                for (int d = 0; d < 7; ++d) s_pos[d] = best < BT ? q0.P[d] : pos_in[d * N + best];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int d = 0; d < 7; ++d) g[d] = s_pos[d];
         }
-        __syncthreads();
-#pragma unroll
-        for (int d = 0; d < 7; ++d) g[d] = s_pos[d];
         g[7] = bv;
     }
-    if (tid == 0) {
-        if (gnew) {
+    if (tid == 0 && (!two || blockIdx.x == 0)) {
+        if (gnew || two) {
 #pragma unroll
-            for (int d = 0; d < 8; ++d) S.gbest[d] = g[d];
+            for (int d = 0; d < 8; ++d) gb_out[d] = g[d];
         }
         if (S.gbest_trace) {
 #pragma unroll
@@ -1920,13 +2049,13 @@ __global__ __launch_bounds__(BT) void k_pso_step(const QpsoSolveDev* __restrict_
         }
         if (S.argmin_trace) S.argmin_trace[iter] = best;
     }
-    if (tid < N) finish_particle(S, tid, q0, g);
-    for (int p = tid + BT; p < N; p += BT) {
+    if (p0 < N) finish_particle(S, p0, q0, g, pos_out);
+    for (int p = tid + BT; p < N && !two; p += BT) {
         Particle q;
-        load_particle(S, p, iter, q);
-        finish_particle(S, p, q, g);
+        load_particle(S, p, iter, false, q);
+        finish_particle(S, p, q, g, pos_out);
     }
-    if (tid == 0) *S.iter = iter + 1;
+    if (tid == 0 && (!two || blockIdx.x == 0)) *S.iter = iter + 1;
 }
 
 }  // namespace
@@ -2000,44 +2129,45 @@ int rf_config_threads(int cfg) { return kRfCfgs[cfg].bt; }
 int rf_config_tile(int cfg) { return kRfCfgs[cfg].cap; }
 bool rf_needs_windows(int cfg, int v_eff) { return v_eff > kRfCfgs[cfg].cap / 6; }
 
-hipError_t init(const QpsoSolveDev* d_solves, int n_solves, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+hipError_t init(const QpsoSolveDev* d_solves, int n_solves, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1, bool two_buffers) {
     if (n_solves <= 0) return hipSuccess;
     if (ev0 || ev1)
-        hipExtLaunchKernelGGL(k_init, dim3(n_solves), dim3(256), 0, st, ev0, ev1, 0, d_solves);
+        hipExtLaunchKernelGGL(k_init, dim3(n_solves), dim3(256), 0, st, ev0, ev1, 0, d_solves, two_buffers ? 1 : 0);
     else
-        hipLaunchKernelGGL(k_init, dim3(n_solves), dim3(256), 0, st, d_solves);
+        hipLaunchKernelGGL(k_init, dim3(n_solves), dim3(256), 0, st, d_solves, two_buffers ? 1 : 0);
     return hipGetLastError();
 }
 
 // With events, the launch stamps them with the dispatch's own start and end
 // (hipExtLaunchKernel), so a timed kernel carries no event-record gaps.
 template <int BT, int CAP, int MODE>
-static void launch_rf_mode(const QpsoSolveDev* d_solves, const QpsoItem* d_items, int n_items, hipStream_t st,
+static void launch_rf_mode(const QpsoSolveDev* d_solves, const QpsoItem* d_items, int n_items, hipStream_t st, int it,
                            hipEvent_t ev0, hipEvent_t ev1) {
     if (ev0 || ev1)
         hipExtLaunchKernelGGL((k_render_fitness<BT, CAP, MODE>), dim3(n_items), dim3(BT), 0, st, ev0, ev1, 0,
-                              d_solves, d_items);
+                              d_solves, d_items, it);
     else
-        hipLaunchKernelGGL((k_render_fitness<BT, CAP, MODE>), dim3(n_items), dim3(BT), 0, st, d_solves, d_items);
+        hipLaunchKernelGGL((k_render_fitness<BT, CAP, MODE>), dim3(n_items), dim3(BT), 0, st, d_solves, d_items, it);
 }
 
 template <int BT, int CAP>
 static void launch_rf(int mode, const QpsoSolveDev* d_solves, const QpsoItem* d_items, int n_items, hipStream_t st,
-                      hipEvent_t ev0, hipEvent_t ev1) {
-    if (mode == 2) launch_rf_mode<BT, CAP, 2>(d_solves, d_items, n_items, st, ev0, ev1);
-    else if (mode == 1) launch_rf_mode<BT, CAP, 1>(d_solves, d_items, n_items, st, ev0, ev1);
-    else launch_rf_mode<BT, CAP, 0>(d_solves, d_items, n_items, st, ev0, ev1);
+                      int it, hipEvent_t ev0, hipEvent_t ev1) {
+    if (mode == 2) launch_rf_mode<BT, CAP, 2>(d_solves, d_items, n_items, st, it, ev0, ev1);
+    else if (mode == 1) launch_rf_mode<BT, CAP, 1>(d_solves, d_items, n_items, st, it, ev0, ev1);
+    else launch_rf_mode<BT, CAP, 0>(d_solves, d_items, n_items, st, it, ev0, ev1);
 }
 
 hipError_t render_fitness(int cfg, int mode, const QpsoSolveDev* d_solves, const QpsoItem* d_items, int n_items,
-                          hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+                          hipStream_t st, hipEvent_t ev0, hipEvent_t ev1, int it) {
     if (n_items <= 0) return hipSuccess;
+    if (it >= 0 && d_items) return hipErrorInvalidValue;  // the step inside the launch takes workgroup b as particle b
     switch (cfg) {
-        case 0: launch_rf<1024, 40448>(mode, d_solves, d_items, n_items, st, ev0, ev1); break;
-        case 1: launch_rf<512, 40448>(mode, d_solves, d_items, n_items, st, ev0, ev1); break;
-        case 2: launch_rf<512, 20224>(mode, d_solves, d_items, n_items, st, ev0, ev1); break;
-        case 3: launch_rf<256, 20224>(mode, d_solves, d_items, n_items, st, ev0, ev1); break;
-        case 4: launch_rf<256, 10112>(mode, d_solves, d_items, n_items, st, ev0, ev1); break;
+        case 0: launch_rf<1024, 40448>(mode, d_solves, d_items, n_items, st, it, ev0, ev1); break;
+        case 1: launch_rf<512, 40448>(mode, d_solves, d_items, n_items, st, it, ev0, ev1); break;
+        case 2: launch_rf<512, 20224>(mode, d_solves, d_items, n_items, st, it, ev0, ev1); break;
+        case 3: launch_rf<256, 20224>(mode, d_solves, d_items, n_items, st, it, ev0, ev1); break;
+        case 4: launch_rf<256, 10112>(mode, d_solves, d_items, n_items, st, it, ev0, ev1); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -2064,9 +2194,15 @@ hipError_t fill_frames(int32_t* d_frames, size_t n_words, hipStream_t st) {
 hipError_t pso_step(const QpsoSolveDev* d_solves, int n_solves, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     if (n_solves <= 0) return hipSuccess;
     if (ev0 || ev1)
-        hipExtLaunchKernelGGL(k_pso_step<256>, dim3(n_solves), dim3(256), 0, st, ev0, ev1, 0, d_solves);
+        hipExtLaunchKernelGGL(k_pso_step<256>, dim3(n_solves), dim3(256), 0, st, ev0, ev1, 0, d_solves, -1);
     else
-        hipLaunchKernelGGL(k_pso_step<256>, dim3(n_solves), dim3(256), 0, st, d_solves);
+        hipLaunchKernelGGL(k_pso_step<256>, dim3(n_solves), dim3(256), 0, st, d_solves, -1);
+    return hipGetLastError();
+}
+
+hipError_t pso_step_two(const QpsoSolveDev* d_solve, int n_particles, int it, hipStream_t st) {
+    if (n_particles <= 0 || it < 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_pso_step<256>, dim3((n_particles + 255) / 256), dim3(256), 0, st, d_solve, it);
     return hipGetLastError();
 }
 
