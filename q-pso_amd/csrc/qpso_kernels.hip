@@ -1845,51 +1845,71 @@ __global__ __launch_bounds__(BT) void k_render_fitness_wrap(const QpsoSolveDev* 
     const int32_t T = ((W * H + 1023) >> 10) << 10;  // NumIters * 1024
     const float rW = rcp((float)W);
     float acc_e[SPT];
+#pragma unroll
+    for (int j = 0; j < SPT; ++j) acc_e[j] = 0.0f;
     uint32_t n_seg = 0, n_tr = 0, n_rend = 0;
     unsigned long long px_f = 0;
-    auto pixel = [&](int32_t t, int32_t& L) {  // false past the last row or outside the buffer
-        const int32_t yb = row_of(t, rW);
-        const int32_t xb = t % W;  // x_bar = tIdxLoop % W_bar
+    auto pixel = [&](int32_t t, int32_t& L) {  // 0: past the last row, 1: in the buffer, 2: outside it
+        const int32_t yb = row_of(t, rW);  // at most one row short of t / W
+        int32_t xb = t - yb * W;
+        if (xb >= W) xb -= W;  // x_bar = tIdxLoop % W_bar
         const int32_t py = minY + yb;
         if (py > maxY) return 0;
         L = wadd(wmul(py, kCols), minX + xb);
         return (uint32_t)L < (uint32_t)kFrame ? 1 : 2;
     };
+    // The pixels' loads set the pace (each waits for the L2 that holds the
+    // atomics' results): U rounds of 2048 pixels go out together, then each
+    // slot sums in increasing t.  One pixel at a time on 256 threads, a
+    // launch of 64 particles at the frame's edge took 490 us, now 150; what
+    // is left waits on the loads one CU can have in flight.
+    constexpr int U = 8 / SPT;
+    for (int32_t base = 0; base < T; base += 2048 * U) {
+        int32_t zr[U][SPT], zk[U][SPT];
+        bool in[U][SPT];
 #pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        acc_e[j] = 0.0f;
-        for (int32_t t = tid + j * BT; t < T; t += 2048) {
-            int32_t L = 0;
-            const int r = pixel(t, L);
-            if (r == 0) break;  // the row index does not decrease with t
-            if (r == 2) continue;
-            ++px_f;
-            const int32_t zr = __hip_atomic_load(buf + L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const int32_t zk = observed_at(S, L);
-            if (zr != QPSO_EMPTY) {
-                ++n_rend;
-                if (zk == 0) {
-                    ++n_tr;
-                } else {
-                    const float e = (float)wsub(zr, zk) * 0.001f;
-                    acc_e[j] = __builtin_fmaf(e, e, acc_e[j]);
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int j = 0; j < SPT; ++j) {
+                const int32_t t = base + 2048 * u + j * BT + tid;
+                int32_t L = 0;
+                in[u][j] = t < T && pixel(t, L) == 1;
+                zr[u][j] = QPSO_EMPTY;
+                zk[u][j] = 0;
+                if (in[u][j]) {
+                    zr[u][j] = __hip_atomic_load(buf + L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    zk[u][j] = observed_at(S, L);
                 }
-            } else if (zk != 0) {
-                ++n_seg;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int j = 0; j < SPT; ++j) {
+                if (!in[u][j]) continue;
+                ++px_f;
+                if (zr[u][j] != QPSO_EMPTY) {
+                    ++n_rend;
+                    if (zk[u][j] == 0) {
+                        ++n_tr;
+                    } else {
+                        const float e = (float)wsub(zr[u][j], zk[u][j]) * 0.001f;
+                        acc_e[j] = __builtin_fmaf(e, e, acc_e[j]);
+                    }
+                } else if (zk[u][j] != 0) {
+                    ++n_seg;
+                }
             }
         }
     }
     __syncthreads();
     // visited pixels are cleared after every read (a pixel visited twice reads
     // its rendered value both times); the others carry their depth
-#pragma unroll
-    for (int j = 0; j < SPT; ++j) {
-        for (int32_t t = tid + j * BT; t < T; t += 2048) {
-            int32_t L = 0;
-            const int r = pixel(t, L);
-            if (r == 0) break;
-            if (r == 1) buf[L] = QPSO_EMPTY;
-        }
+    for (int32_t t = tid; t < T; t += BT) {
+        int32_t L = 0;
+        const int r = pixel(t, L);
+        if (r == 0) break;  // the row index does not decrease with t
+        if (r == 1) buf[L] = QPSO_EMPTY;
     }
 
     // FitnessReductionBallot's halving tree (main.h:1522-1573)
@@ -2177,10 +2197,10 @@ hipError_t render_fitness_wrap(const QpsoSolveDev* d_solves, const QpsoItem* d_i
                                hipEvent_t ev0, hipEvent_t ev1) {
     if (n_items <= 0) return hipSuccess;
     if (ev0 || ev1)
-        hipExtLaunchKernelGGL(k_render_fitness_wrap<256>, dim3(n_items), dim3(256), 0, st, ev0, ev1, 0, d_solves,
+        hipExtLaunchKernelGGL(k_render_fitness_wrap<1024>, dim3(n_items), dim3(1024), 0, st, ev0, ev1, 0, d_solves,
                               d_items);
     else
-        hipLaunchKernelGGL(k_render_fitness_wrap<256>, dim3(n_items), dim3(256), 0, st, d_solves, d_items);
+        hipLaunchKernelGGL(k_render_fitness_wrap<1024>, dim3(n_items), dim3(1024), 0, st, d_solves, d_items);
     return hipGetLastError();
 }
 
