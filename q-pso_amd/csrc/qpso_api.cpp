@@ -211,6 +211,17 @@ struct qpso_ctx {
     // ran it, with no wait (hipFree waits for the whole device); freed
     // memory stays in the pool for reuse until the context is destroyed
     hipMemPool_t pool = nullptr;
+    // Host copies of the calls on `stream`: a call's inputs go up and its
+    // results come down as one copy each through pinned memory (a pageable
+    // copy takes several times a pinned one's time, and a solve had three
+    // each way).  `work`: poses in, boxes and fitness out of
+    // qpso_solve_eval_poses.  Both are used under `mu` by calls that end
+    // synchronised, grow to the largest call (at most a frame's crop, 65,535
+    // particles' poses) and go with the context.
+    char* stage = nullptr;
+    size_t stage_bytes = 0;
+    char* work = nullptr;
+    size_t work_bytes = 0;
 };
 
 struct qpso_solve {
@@ -265,6 +276,22 @@ int validate(const qpso_cluster* cl, const qpso_params* p) {
 hipError_t copy_on(hipStream_t st, void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, kind, st);
     return e == hipSuccess ? hipStreamSynchronize(st) : e;
+}
+
+// Pinned staging of at least this many bytes (null if there is none to be had).
+char* stage_for(qpso_ctx* ctx, size_t bytes) {
+    if (bytes <= ctx->stage_bytes) return ctx->stage;
+    if (ctx->stage) hipHostFree(ctx->stage);
+    ctx->stage = nullptr;
+    ctx->stage_bytes = 0;
+    const size_t n = align_up(std::max(bytes, size_t(64) << 10), size_t(64) << 10);
+    if (hipHostMalloc(reinterpret_cast<void**>(&ctx->stage), n) != hipSuccess) {
+        hipGetLastError();
+        ctx->stage = nullptr;
+        return nullptr;
+    }
+    ctx->stage_bytes = n;
+    return ctx->stage;
 }
 
 // A solve arena: from the context's pool in the order of its stream (the
@@ -373,20 +400,45 @@ int result_from(const ResultWords& w, qpso_result* out) {
     return status;
 }
 
-int read_result_status(qpso_solve* s, qpso_result* out, hipStream_t st) {
-    ResultWords w{};
-    if (copy_result(s, &w, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return QPSO_E_HIP;
-    return result_from(w, out);
+// The results of n solves whose work lies on the context's stream: one copy a
+// solve (gbest, iteration, flags and counters lie together), one wait.
+// Caller holds ctx->mu.
+int read_results(qpso_ctx* ctx, int n, qpso_solve* const* solves, qpso_result* out) {
+    const hipStream_t st = ctx->stream;
+    constexpr size_t kWords = 1024;  // a solve's part of the staging
+    char* h = stage_for(ctx, kWords * n);
+    if (!h) return QPSO_E_NOMEM;
+    for (int i = 0; i < n; ++i) {
+        const ArenaLayout& L = solves[i]->L;
+        if (hipMemcpyAsync(h + kWords * i, solves[i]->arena + L.gbest, L.counters + 24 - L.gbest, hipMemcpyDeviceToHost,
+                           st) != hipSuccess)
+            return QPSO_E_HIP;
+    }
+    if (hipStreamSynchronize(st) != hipSuccess) return QPSO_E_HIP;
+    int rc = QPSO_OK;
+    for (int i = 0; i < n; ++i) {
+        const ArenaLayout& L = solves[i]->L;
+        ResultWords w{};
+        const char* p = h + kWords * i;
+        std::memcpy(w.g, p, sizeof(w.g));
+        std::memcpy(&w.flags, p + (L.flags - L.gbest), sizeof(w.flags));
+        std::memcpy(w.c, p + (L.counters - L.gbest), sizeof(w.c));
+        const int r = result_from(w, out ? &out[i] : nullptr);
+        if (r && !rc) rc = r;
+    }
+    return rc;
 }
 
-int read_result(qpso_solve* s, qpso_result* out, hipStream_t st) {
-    const int rc = read_result_status(s, out, st);
+int read_results_err(qpso_ctx* ctx, int n, qpso_solve* const* solves, qpso_result* out) {
+    const int rc = read_results(ctx, n, solves, out);
     switch (rc) {
         case QPSO_OK: return QPSO_OK;
-        case QPSO_E_STALE: return set_err(s->ctx, rc, "stale-pixel list overflow");
-        default: return set_err(s->ctx, rc, "result readback failed, or a render kernel launched without mesh windows");
+        case QPSO_E_STALE: return set_err(ctx, rc, "stale-pixel list overflow");
+        default: return set_err(ctx, rc, "result readback failed, or a render kernel launched without mesh windows");
     }
 }
+
+int read_result(qpso_solve* s, qpso_result* out) { return read_results_err(s->ctx, 1, &s, out); }
 
 bool needs_windows(const qpso_solve* s, int cfg) { return qpso_launch::rf_needs_windows(cfg, s->h.V_eff); }
 
@@ -552,6 +604,8 @@ int qpso_destroy(qpso_ctx* ctx) {
     invalidate_plan(ctx);
     for (auto& kv : ctx->meshes) free_mesh(kv.second);
     for (auto& kv : ctx->rand_cache) hipFree(kv.second.d);
+    if (ctx->stage) hipHostFree(ctx->stage);
+    if (ctx->work) hipFree(ctx->work);
     if (ctx->pool) {
         hipDeviceSynchronize();
         hipMemPoolDestroy(ctx->pool);
@@ -663,11 +717,17 @@ int create_solve(qpso_ctx* ctx, uint32_t mesh_id, const qpso_cluster* cl, const 
     qpso_host::build_crop(cl->depth, kCols, cl->rect, crop, rows);
     hipStream_t st = ctx->stream;
     int rc = QPSO_OK;
-    if (hipMemcpyAsync(A + s->L.obs, crop.data(), crop.size() * 2, hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipMemcpyAsync(A + s->L.obs_rows, rows.data(), rows.size() * 2, hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipMemcpyAsync(s->d_desc, &s->h, sizeof(QpsoSolveDev), hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-        rc = set_err(ctx, QPSO_E_HIP, "solve upload failed");
+    // the descriptor, the crop and its rows open the arena: one copy
+    const size_t up = s->L.obs_rows + rows.size() * 2;
+    if (char* h = stage_for(ctx, up)) {
+        std::memcpy(h + s->L.desc, &s->h, sizeof(QpsoSolveDev));
+        std::memcpy(h + s->L.obs, crop.data(), crop.size() * 2);
+        std::memcpy(h + s->L.obs_rows, rows.data(), rows.size() * 2);
+        if (copy_on(st, A, h, up, hipMemcpyHostToDevice) != hipSuccess)
+            rc = set_err(ctx, QPSO_E_HIP, "solve upload failed");
+    } else {
+        rc = set_err(ctx, QPSO_E_NOMEM, "no pinned memory for the upload");
+    }
     if (rc) {
         free_arena(ctx, s->arena, st);
         hipStreamSynchronize(st);
@@ -720,7 +780,7 @@ int qpso_solve_run(qpso_solve* s, qpso_result* out) {
     std::lock_guard<std::mutex> g(ctx->mu);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     if (int r = run_solve_graph(s, ctx->stream)) return r;
-    return read_result(s, out, ctx->stream);
+    return read_result(s, out);
 }
 
 int qpso_solve_run_reference_launches(qpso_solve* s, qpso_result* out) {
@@ -769,7 +829,7 @@ int qpso_solve_run_reference_launches(qpso_solve* s, qpso_result* out) {
     }
     cleanup();
     if (e != hipSuccess) return set_err(ctx, QPSO_E_HIP, std::string("reference-shaped run: ") + hipGetErrorString(e));
-    return read_result(s, out, st);
+    return read_result(s, out);
 }
 
 int qpso_solve_run_timed(qpso_solve* s, qpso_result* out, qpso_timing* tm) {
@@ -809,7 +869,7 @@ int qpso_solve_run_timed(qpso_solve* s, qpso_result* out, qpso_timing* tm) {
     }
     tm->ms_solve = span(0, n_ev - 1);
     tm->launches = I;
-    return read_result(s, out, st);
+    return read_result(s, out);
 }
 
 int qpso_estimate_pose(qpso_ctx* ctx, uint32_t mesh_id, const qpso_cluster* cl, const qpso_params* p,
@@ -823,7 +883,7 @@ int qpso_estimate_pose(qpso_ctx* ctx, uint32_t mesh_id, const qpso_cluster* cl, 
         std::lock_guard<std::mutex> g(ctx->mu);
         r = hipSetDevice(ctx->device) == hipSuccess ? launch_solve(s, ctx->stream)
                                                    : set_err(ctx, QPSO_E_HIP, "hipSetDevice failed");
-        if (!r) r = read_result(s, out, ctx->stream);
+        if (!r) r = read_result(s, out);
     }
     qpso_solve_destroy(s);
     return r;
@@ -961,34 +1021,41 @@ int qpso_solve_eval_poses(qpso_solve* s, int n, const float* poses, float* fit, 
     std::lock_guard<std::mutex> g(ctx->mu);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    const int N = s->h.N;
-    char* A = s->arena;
-    for (int d = 0; d < 7; ++d)
-        HIP_TRY(ctx, hipMemcpyAsync(A + s->L.pos + sizeof(float) * (size_t)d * N, poses + (size_t)d * n,
-                                    sizeof(float) * n, hipMemcpyHostToDevice, st));
-    HIP_TRY(ctx, hipMemsetAsync(A + s->L.iter, 0, sizeof(int32_t), st));
-    HIP_TRY(ctx, hipMemsetAsync(A + s->L.flags, 0, sizeof(int32_t), st));
-    HIP_TRY(ctx, hipMemsetAsync(A + s->L.cnt0, 0, sizeof(int32_t) * N, st));
-    HIP_TRY(ctx, hipMemsetAsync(A + s->L.counters, 0, sizeof(unsigned long long) * 3, st));
+    // workspace: the evaluation's descriptor and the poses (up in one copy),
+    // the fitness and the boxes (down in one)
+    const size_t o_pos = align_up(sizeof(QpsoSolveDev), 256), up = o_pos + sizeof(float) * 7 * (size_t)n;
+    const size_t o_fit = align_up(up, 256), o_box = align_up(o_fit + sizeof(float) * (size_t)n, 16);
+    const size_t total = o_box + sizeof(int32_t) * 4 * (size_t)n;
+    if (total > ctx->work_bytes) {
+        if (ctx->work) hipFree(ctx->work);
+        ctx->work = nullptr;
+        ctx->work_bytes = 0;
+        const size_t bytes = align_up(total, size_t(64) << 10);
+        if (hipMalloc(reinterpret_cast<void**>(&ctx->work), bytes) != hipSuccess) {
+            ctx->work = nullptr;
+            return set_err(ctx, QPSO_E_NOMEM, "pose evaluation workspace");
+        }
+        ctx->work_bytes = bytes;
+    }
+    char* const W = ctx->work;
+    char* const h = stage_for(ctx, total);
+    if (!h) return set_err(ctx, QPSO_E_NOMEM, "no pinned memory for the poses");
     int32_t* d_frames = nullptr;
-    int32_t* d_aabb = nullptr;
-    QpsoSolveDev* d_tmp = nullptr;
-    auto cleanup = [&]() {
-        hipStreamSynchronize(st);
-        if (d_frames) hipFree(d_frames);
-        if (d_aabb) hipFree(d_aabb);
-        if (d_tmp) hipFree(d_tmp);
-    };
     QpsoSolveDev tmp = s->h;
+    tmp.fit = reinterpret_cast<float*>(W + o_fit);
+    tmp.dbg_aabb = reinterpret_cast<int32_t*>(W + o_box);
     if (frames) {
-        if (hipMalloc(&d_frames, sizeof(int32_t) * (size_t)n * kFrame) != hipSuccess) { cleanup(); return QPSO_E_NOMEM; }
+        if (hipMalloc(&d_frames, sizeof(int32_t) * (size_t)n * kFrame) != hipSuccess)
+            return set_err(ctx, QPSO_E_NOMEM, "frame dump allocation failed");
         hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(d_frames), QPSO_EMPTY, (size_t)n * kFrame, st);
         tmp.dbg_frames = d_frames;
     }
-    if (hipMalloc(&d_aabb, sizeof(int32_t) * 4 * (size_t)n) != hipSuccess) { cleanup(); return QPSO_E_NOMEM; }
-    tmp.dbg_aabb = d_aabb;
-    if (hipMalloc(&d_tmp, sizeof(QpsoSolveDev)) != hipSuccess) { cleanup(); return QPSO_E_NOMEM; }
-    hipError_t e = hipMemcpyAsync(d_tmp, &tmp, sizeof(tmp), hipMemcpyHostToDevice, st);
+    std::memcpy(h, &tmp, sizeof(tmp));
+    std::memcpy(h + o_pos, poses, sizeof(float) * 7 * (size_t)n);
+    const QpsoSolveDev* const d_tmp = reinterpret_cast<const QpsoSolveDev*>(W);
+    hipError_t e = hipMemcpyAsync(W, h, up, hipMemcpyHostToDevice, st);
+    // the poses become the solve's first n particles, its iteration 0
+    if (e == hipSuccess) e = qpso_launch::eval_begin(d_tmp, reinterpret_cast<const float*>(W + o_pos), n, s->h.N, st);
     if (s->h.wrap) {  // the particles' own buffers start empty too
         if (e == hipSuccess) e = qpso_launch::fill_frames(s->h.frames, (size_t)n * kFrame, st);
         if (e == hipSuccess) e = qpso_launch::render_fitness_wrap(d_tmp, nullptr, n, st);
@@ -996,13 +1063,15 @@ int qpso_solve_eval_poses(qpso_solve* s, int n, const float* poses, float* fit, 
         // frames come from their own instantiation (it handles every mesh)
         e = qpso_launch::render_fitness(s->rf_cfg, frames ? 2 : needs_windows(s, s->rf_cfg) ? 1 : 0, d_tmp, nullptr, n, st);
     }
-    if (e == hipSuccess && fit) e = hipMemcpyAsync(fit, A + s->L.fit, sizeof(float) * n, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess && aabb) e = hipMemcpyAsync(aabb, d_aabb, sizeof(int32_t) * 4 * n, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(h + o_fit, W + o_fit, total - o_fit, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess && frames)
         e = hipMemcpyAsync(frames, d_frames, sizeof(int32_t) * (size_t)n * kFrame, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    cleanup();
+    const hipError_t e2 = hipStreamSynchronize(st);  // whatever was queued has ended
+    if (e == hipSuccess) e = e2;
+    if (d_frames) hipFree(d_frames);
     if (e != hipSuccess) return set_err(ctx, QPSO_E_HIP, std::string("eval_poses: ") + hipGetErrorString(e));
+    if (fit) std::memcpy(fit, h + o_fit, sizeof(float) * (size_t)n);
+    if (aabb) std::memcpy(aabb, h + o_box, sizeof(int32_t) * 4 * (size_t)n);
     return QPSO_OK;
 }
 
@@ -1155,12 +1224,7 @@ int qpso_solve_run_batch(qpso_ctx* ctx, int n, qpso_solve* const* solves, qpso_r
         if (e != hipSuccess) { invalidate_plan(ctx); return set_err(ctx, QPSO_E_HIP, "graph instantiate failed"); }
     }
     HIP_TRY(ctx, hipGraphLaunch(P.exec, st));
-    int rc = QPSO_OK;
-    for (int i = 0; i < n; ++i) {
-        int r = read_result(solves[i], out ? &out[i] : nullptr, st);
-        if (r && !rc) rc = r;
-    }
-    return rc;
+    return read_results_err(ctx, n, solves, out);
 }
 
 }  // extern "C"

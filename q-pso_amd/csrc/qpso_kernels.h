@@ -36,6 +36,9 @@ hipError_t render_fitness(int cfg, int mode, const QpsoSolveDev* d_solves, const
 // full per-particle buffers in device memory, linear-index wrap).
 hipError_t render_fitness_wrap(const QpsoSolveDev* d_solves, const QpsoItem* d_items, int n_items, hipStream_t st,
                                hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// A pose evaluation's start: n poses ([7][n]) into the solve's first particles;
+// iteration, flags, work counters and all carried-pixel counts to zero.
+hipError_t eval_begin(const QpsoSolveDev* d_solve, const float* poses, int n, int n_particles, hipStream_t st);
 // Sets n_words depth words to the empty value 60000 (a kernel, not a memset).
 hipError_t fill_frames(int32_t* d_frames, size_t n_words, hipStream_t st);
 // argmin + pbest/gbest + particle update, one workgroup per solve.

@@ -2114,6 +2114,31 @@ hipError_t scratch_address(int device, void** ptr) {
     return hipSuccess;
 }
 
+// ------------------------------------------------------------------------
+// start of a pose evaluation
+// ------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_eval_begin(const QpsoSolveDev* __restrict__ solve, const float* __restrict__ poses,
+                                                    int n) {
+    const QpsoSolveDev& S = *solve;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) {
+#pragma unroll
+        for (int d = 0; d < 7; ++d) S.pos[d * S.N + i] = poses[d * n + i];
+    }
+    if (i < S.N) S.stale_cnt[0][i] = 0;
+    if (i == 0) {
+        *S.iter = 0;
+        *S.flags = 0;
+        S.counters[0] = S.counters[1] = S.counters[2] = 0;
+    }
+}
+
+hipError_t eval_begin(const QpsoSolveDev* d_solve, const float* poses, int n, int n_particles, hipStream_t st) {
+    if (n <= 0 || n > n_particles) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_eval_begin, dim3((n_particles + 255) / 256), dim3(256), 0, st, d_solve, poses, n);
+    return hipGetLastError();
+}
+
 // Per crop row, the number of observed (non-zero) pixels left of each column
 // ((rw + 1) counts a row), one thread per row.
 __global__ __launch_bounds__(256) void k_obs_rows(const uint16_t* __restrict__ crop, uint16_t* __restrict__ rows,
