@@ -405,6 +405,7 @@ struct RfLds {
     int32_t s_nqb;       // big faces queued
     int32_t s_take;      // next big face to hand to a wave
     int32_t s_later[3];  // a face of the window reaches later bands (slot: windows drawn mod 3)
+    int32_t s_next[3];   // groups of face batches handed out in the window (the same slot)
     uint32_t s_cnt[3];   // seg, tr, n_rendered
     unsigned long long s_px[2];
     float s_pose[7];     // the particle's pose, from the PSO step inside the launch
@@ -427,6 +428,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     int32_t& s_nqb = sh.s_nqb;
     int32_t& s_take = sh.s_take;
     int32_t* const s_later = sh.s_later;
+    int32_t* const s_next = sh.s_next;
     uint32_t* const s_cnt = sh.s_cnt;
     unsigned long long* const s_px = sh.s_px;
 
@@ -502,6 +504,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         s_stale[2] = INT32_MAX; s_stale[3] = INT32_MIN;
         s_degen = 0; s_nstale = 0; s_nq = 0; s_nqb = 0; s_take = 0;
         s_later[0] = s_later[1] = s_later[2] = 0;
+        s_next[0] = s_next[1] = s_next[2] = 0;
         s_cnt[0] = s_cnt[1] = s_cnt[2] = 0;
         s_px[0] = s_px[1] = 0;
     }
@@ -534,18 +537,23 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     constexpr int kGroup = WIN ? 2 : 1;
     constexpr int kRing = 64 * (kGroup + 1);
     constexpr int kFixed = kQCap + 4 * kBQCap + (BT / 64) * kRing + 4;  // queues, rings, alignment
-    constexpr int kMinVC = CAP / 12 > qpso_host::kRunVerts ? CAP / 12 : qpso_host::kRunVerts;  // shortest window
-    constexpr int kMinTile = 2048 + CAP / 8;  // a row of the frame with its lines, and the later bits
+    // shortest window: shorter ones cost more barriers than a band more
+    // (100k faces on 512 threads and 20,224 words: 476 ms a solve with CAP / 12,
+    // 443 with CAP / 6, 471 with CAP / 3)
+    constexpr int kMinVC = CAP / 6 > qpso_host::kRunVerts ? CAP / 6 : qpso_host::kRunVerts;
+    const int32_t n_lw = (Fe + 63) >> 6;           // later bits: 64-bit words
+    const int32_t l_words = 2 * n_lw <= CAP / 8 ? 2 * n_lw : 0;
+    const int32_t min_tile = 2048 + l_words;       // a row of the frame with its lines, and the later bits
     const int32_t rect_words = [&] {  // a band of the whole rect
         const int32_t rw = S.rect[2] - S.rect[0], rh = S.rect[3] - S.rect[1];
         return rw * rh + rh * (((rw + 31) >> 5) + 1) + rw + 8;
     }();
     // compile-time true without windows
-    const bool cached = !WIN || Ve <= max(2 * kWin, CAP - kFixed - max(rect_words / 2 + 1024, kMinTile));
+    const bool cached = !WIN || Ve <= max(2 * kWin, CAP - kFixed - max(rect_words / 2 + 1024, min_tile));
     const bool runs = WIN && !cached && S.n_runs > 0 && S.n_runs * 256 <= Fe;  // runs of 256 faces on average
     bool pack = cached || runs;
     int VC = cached ? Ve : 2 * kWin;  // cache capacity in vertices
-    const bool zc = cached && max(rect_words, kMinTile) <= CAP - kFixed - 2 * VC;
+    const bool zc = cached && max(rect_words, min_tile) <= CAP - kFixed - 2 * VC;
     uint32_t* __restrict__ vP = reinterpret_cast<uint32_t*>(lds);  // X | Y << 16
     float* __restrict__ vZ = reinterpret_cast<float*>(lds + VC);
     int32_t vbase = 0;  // vertex index of cache entry 0
@@ -731,15 +739,14 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     // not fit beside the rest
     const int32_t TH = has_tile ? ty1 - ty0 : 0;
     const int32_t region = TH * (MW + 1) + (DW > 0 ? DW * (dy1 - dy0) : 0);
-    const int32_t n_lw = (Fe + 63) >> 6;
     const bool win = WIN && runs && pack;
     int32_t v_words = !pack ? 0 : zc ? 2 * VC : VC;
     bool lbits = region + TW + 8 > CAP - kFixed - (win ? kMinVC : v_words);
-    lbits = lbits && 2 * n_lw <= CAP / 8;
+    lbits = lbits && l_words > 0;
     if (win) {
         // the largest window, up to 2 kWin, that costs no band: projecting
         // and culling a band's windows again costs more than shorter windows
-        const int32_t room = CAP - kFixed - (lbits ? 2 * n_lw : 0) - TW - 8;
+        const int32_t room = CAP - kFixed - (lbits ? l_words : 0) - TW - 8;
         int32_t vw = room - region;
         for (int32_t nb = 2; vw < kMinVC && nb <= 16; ++nb) vw = room - (region + nb - 1) / nb - DW - MW - 1;
         VC = min(2 * kWin, max(vw, kMinVC));
@@ -762,7 +769,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     // 128-bit fills
     const int32_t l_off = ((int32_t)(rings - lds) + (BT / 64) * kRing + 1) & ~1;
     unsigned long long* const later = reinterpret_cast<unsigned long long*>(lds + l_off);
-    const int32_t tile_off = (l_off + (lbits ? 2 * n_lw : 0) + 3) & ~3;
+    const int32_t tile_off = (l_off + (lbits ? l_words : 0) + 3) & ~3;
     int32_t* __restrict__ tile = lds + tile_off;
     const int32_t tcap = CAP - tile_off;
 
@@ -1006,6 +1013,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         const bool more = b1 < ty1;  // bands follow
         if (lbits && first && more)
             for (int i = tid; i < n_lw; i += BT) later[i] = 0ull;
+        if (WIN && tid == 0) s_next[wslot] = 0;
         {
             typedef int32_t v4i __attribute__((ext_vector_type(4)));
             v4i* t4 = reinterpret_cast<v4i*>(tile);
@@ -1213,19 +1221,32 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         // is one word of the later bits.  kGroup batches are culled together,
         // the face entries of the next group in flight (lanes outside the
         // window load one of the window's): with one batch in flight the
-        // loads' latency set the pace of the cull.
+        // loads' latency set the pace of the cull.  The waves of a large
+        // mesh take groups from a counter, each the one after its next ahead
+        // of time: with fixed shares the older waves, which the SIMDs prefer,
+        // waited at the barrier while the younger ones ran on with nothing to
+        // hide their latencies (50k faces, 128 particles: 76 -> 70 us a
+        // launch; 100k, 2,048: 1,857 -> 1,758).  A mesh of a few batches a
+        // wave keeps fixed shares (10k faces: 72.5 us, 74.8 with the counter).
         int cnt = 0;  // faces waiting in the ring (wave-uniform), last in first out
         uint64_t any_later = 0;
-        int base = __builtin_amdgcn_readfirstlane((f_lo & ~63) + tid - lane);
+        constexpr int kSpan = 64 * kGroup;
+        const int f_0 = f_lo & ~63, n_groups = (f_hi - f_0 + kSpan - 1) / kSpan;
+        auto grab = [&] { return WIN && lane == 0 ? atomicAdd(&s_next[wslot], 1) : 0; };
+        int gi = __builtin_amdgcn_readfirstlane(tid >> 6), got = grab();
         const bool fetch = pack && (first || !lbits);  // every face of [f_lo, f_hi), from the cache
         qv2 nx[kGroup];
 #pragma unroll
         for (int g = 0; g < kGroup; ++g) nx[g] = qv2{0, 0};
-        if (fetch) {
+        if (fetch && gi < n_groups) {
 #pragma unroll
-            for (int g = 0; g < kGroup; ++g) nx[g] = load_ref(faces, min(max(base + g * BT + lane, f_lo), f_hi - 1));
+            for (int g = 0; g < kGroup; ++g)
+                nx[g] = load_ref(faces, min(max(f_0 + gi * kSpan + g * 64 + lane, f_lo), f_hi - 1));
         }
-        for (;; base += kGroup * BT) {
+        while (gi < n_groups) {
+            const int base = f_0 + gi * kSpan;
+            const int ng = BT / 64 + (WIN ? __builtin_amdgcn_readfirstlane(got) : gi);
+            if (ng < n_groups) got = grab();
             // per batch of the group: the faces to draw in this band, and
             // those that reach below it
             uint64_t m[kGroup], lm[kGroup];
@@ -1241,13 +1262,14 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                     pv[g][1] = vP[((x >> 16) - vb) & 0xffffu];
                     pv[g][2] = vP[(y - vb) & 0xffffu];
                 }
-                if (base + kGroup * BT < f_hi) {
+                if (ng < n_groups) {
 #pragma unroll
-                    for (int g = 0; g < kGroup; ++g) nx[g] = load_ref(faces, min(base + (kGroup + g) * BT + lane, f_hi - 1));
+                    for (int g = 0; g < kGroup; ++g)
+                        nx[g] = load_ref(faces, min(f_0 + ng * kSpan + g * 64 + lane, f_hi - 1));
                 }
 #pragma unroll
                 for (int g = 0; g < kGroup; ++g) {
-                    const int i = base + g * BT + lane;
+                    const int i = base + g * 64 + lane;
                     bool keep, down;
                     const bool reach = cull_packed(pv[g][0], pv[g][1], pv[g][2], lo2, hi2, b1w, keep, down);
                     const uint64_t in = __ballot((uint32_t)(i - f_lo) < (uint32_t)(f_hi - f_lo)) & __ballot(reach);
@@ -1257,7 +1279,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             } else {
 #pragma unroll 1
                 for (int g = 0; g < kGroup; ++g) {
-                    const int bg = base + g * BT, i = bg + lane;
+                    const int bg = base + g * 64, i = bg + lane;
                     uint64_t mg = 0, lg = 0;
                     const uint64_t todo = bg >= f_hi ? 0ull : first || !lbits ? ~0ull : uniform64(later[bg >> 6]);
                     if (direct) {
@@ -1292,10 +1314,10 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
 #pragma unroll
                 for (int g = 0; g < kGroup; ++g) {
                     any_later |= lm[g];
-                    if (lbits && !direct && base + g * BT < f_hi && lane == 0) {
+                    if (lbits && !direct && base + g * 64 < f_hi && lane == 0) {
                         // a window's first and last word is shared with its neighbours
-                        if (!first) later[(base + g * BT) >> 6] = lm[g];
-                        else if (lm[g] != 0ull) atomicOr(&later[(base + g * BT) >> 6], (unsigned long long)lm[g]);
+                        if (!first) later[(base + g * 64) >> 6] = lm[g];
+                        else if (lm[g] != 0ull) atomicOr(&later[(base + g * 64) >> 6], (unsigned long long)lm[g]);
                     }
                 }
             }
@@ -1303,18 +1325,18 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             for (int g = 0; g < kGroup; ++g) {
                 if (__builtin_amdgcn_inverse_ballot_w64(m[g]))
                     ring[__builtin_amdgcn_mbcnt_hi((uint32_t)(m[g] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[g], (uint32_t)cnt))] =
-                        base + g * BT + lane;
+                        base + g * 64 + lane;
                 cnt += __popcll(m[g]);
             }
             __builtin_amdgcn_wave_barrier();
-            const bool last = base + kGroup * BT >= f_hi;
+            const bool last = ng >= n_groups;
             while (cnt >= 64 || (last && cnt > 0)) {
                 const int n = min(cnt, 64);
                 cnt -= n;
                 if (lane < n) draw(ring[cnt + lane]);
                 __builtin_amdgcn_wave_barrier();
             }
-            if (last) break;
+            gi = ng;
         }
         if (!win || direct) break;  // one pass over the faces; the queues follow
         // windows: the queued faces wait for the band's end (they are
@@ -1324,7 +1346,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         // slot (last read two windows ago, before the previous barrier) is
         // cleared before it.
         if (any_later != 0ull && lane == 0) s_later[wslot] = 1;
-        if (tid == 0) s_later[wslot == 2 ? 0 : wslot + 1] = 0;
+        if (tid == 0) s_later[wslot == 2 ? 0 : wslot + 1] = s_next[wslot == 2 ? 0 : wslot + 1] = 0;
         __syncthreads();
         if (wi < 64 && s_later[wslot] == 0) wmask &= ~(1ull << wi);
         wslot = wslot == 2 ? 0 : wslot + 1;
