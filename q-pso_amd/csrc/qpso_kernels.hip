@@ -590,8 +590,10 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                 float a, b;
                 ok = ok & vertex_fast(pose, x, y, z, cam16, a, b, Z);
                 xy = pack_fast(a, b);
-                fxl = min_num(fxl, a); fxh = max_num(fxh, a);
-                fyl = min_num(fyl, b); fyh = max_num(fyh, b);
+                // a coordinate that is no number (a quaternion or a mesh of
+                // 1e20 overflows in X and Y alone) fails the range test too
+                fxl = min_nan(fxl, a); fxh = max_nan(fxh, a);
+                fyl = min_nan(fyl, b); fyh = max_nan(fyh, b);
             }
             if (!WIN || v < VC) {  // windows: the one from vertex 0, kept if every coordinate fits
                 if (pack) vP[v] = xy;

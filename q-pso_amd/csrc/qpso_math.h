@@ -212,14 +212,17 @@ struct Cam {
     double fx, fy, cx, cy;
 };
 
-// The rotation's 2 (q x v) takes its factor into the constants: doubling is
-// exact.
+// A vertex in the camera's frame.  kBounded (fast_inputs): the rotation's
+// 2 (q x v) takes its factor into the constants, where doubling is exact; it is
+// not for a quaternion that overflows doubled.
+template <bool kBounded>
 QD void to_camera(const float pose[7], float vx, float vy, float vz, float& px, float& py, float& pz) {
     const float q0 = pose[3], q1 = pose[4], q2 = pose[5], q3 = pose[6];
-    const float d1 = 2.0f * q1, d2 = 2.0f * q2, d3 = 2.0f * q3;
-    const float t0 = __builtin_fmaf(d2, vz, -(d3 * vy));
-    const float t1 = __builtin_fmaf(-d1, vz, d3 * vx);
-    const float t2 = __builtin_fmaf(d1, vy, -(d2 * vx));
+    const float a = kBounded ? 2.0f : 1.0f, b = kBounded ? 1.0f : 2.0f;
+    const float d1 = a * q1, d2 = a * q2, d3 = a * q3;
+    const float t0 = b * __builtin_fmaf(d2, vz, -(d3 * vy));
+    const float t1 = b * __builtin_fmaf(-d1, vz, d3 * vx);
+    const float t2 = b * __builtin_fmaf(d1, vy, -(d2 * vx));
     const float k0 = __builtin_fmaf(q2, t2, -(q3 * t1));
     const float k1 = __builtin_fmaf(-q1, t2, q3 * t0);
     const float k2 = __builtin_fmaf(q1, t1, -(q2 * t0));
@@ -234,7 +237,7 @@ QD void to_camera(const float pose[7], float vx, float vy, float vz, float& px, 
 QD void project(const float pose[7], float vx, float vy, float vz, const Cam& c,
                 float& u, float& v, float& Z) {
     float px, py, pz;
-    to_camera(pose, vx, vy, vz, px, py, pz);
+    to_camera<false>(pose, vx, vy, vz, px, py, pz);
     const float r = rcp_any(pz);
     u = (float)__builtin_fma(c.fx, (double)(px * r), c.cx);
     v = (float)__builtin_fma(c.fy, (double)(py * r), c.cy);
@@ -252,7 +255,7 @@ constexpr float kFastLimit = 0x1p22f;
 constexpr float kRound = 0x1.8p23f;
 QD bool vertex_fast(const float pose[7], float vx, float vy, float vz, const Cam16& c, float& x, float& y, float& Z) {
     float px, py, pz, e;
-    to_camera(pose, vx, vy, vz, px, py, pz);
+    to_camera<true>(pose, vx, vy, vz, px, py, pz);
     const float r = rcp_newton(pz, e);
     x = (float)__builtin_fma(c.fx, (double)(px * r), c.cx);
     y = (float)__builtin_fma(c.fy, (double)(py * r), c.cy);
@@ -271,6 +274,17 @@ QD float max_num(float a, float b) {
     asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
+// and the forms that hand a NaN operand on, at the same rate
+QD float min_nan(float a, float b) {
+    float r;
+    asm("v_minimum3_f32 %0, %1, %2, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+QD float max_nan(float a, float b) {
+    float r;
+    asm("v_maximum3_f32 %0, %1, %2, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 // X | Y << 16 of such coordinates
 QD uint32_t pack_fast(float x, float y) {
     return __builtin_amdgcn_perm(__float_as_uint(y + kRound), __float_as_uint(x + kRound), 0x05040100u);
@@ -278,7 +292,9 @@ QD uint32_t pack_fast(float x, float y) {
 // whether the pose and the camera are numbers that vertex_fast takes
 QD bool fast_inputs(const float pose[7], const Cam& c) {
     const double m = __builtin_fabs(c.fx) + __builtin_fabs(c.fy) + __builtin_fabs(c.cx) + __builtin_fabs(c.cy);
-    const float p = __builtin_fabsf(pose[0]) + __builtin_fabsf(pose[1]);
+    float p = 0.0f;
+#pragma unroll
+    for (int d = 0; d < 7; ++d) p += __builtin_fabsf(pose[d]);
     return m < 1e30 && p < 1e30f;
 }
 
