@@ -173,7 +173,8 @@ int qpso_solve_run_reference_launches(qpso_solve* s, qpso_result* out);
 /* qpso_solve_run with every kernel timed (the reference's myTimer brackets,
  * main.cu:1617-1733, per kernel): each launch stamps a start and a stop event
  * with its own dispatch, so the figures are kernel durations without event
- * records between the kernels. */
+ * records between the kernels.  The PSO step has a launch of its own here
+ * (qpso_solve_run may do it inside the next render launch; equal results). */
 typedef struct {
     double ms_solve;          /* start of InitQPSO to the end of the last kernel */
     double ms_render_fitness; /* sum over the I render+fitness launches */
