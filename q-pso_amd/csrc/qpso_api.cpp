@@ -57,6 +57,7 @@ struct Mesh {
     QpsoFaceIdx* faces = nullptr;  // vertex indices per face, face order [F]
     float* corners = nullptr;      // [F][3][4]: a face's corners (x, y, z, vertex index bits), 16 bytes each
     uint32_t F = 0, V = 0;
+    bool bounded = false;            // every coordinate is below QPSO_MESH_BOUND in magnitude
     std::vector<uint32_t> v_prefix;  // unique vertices referenced by faces [0, f+1)
     int32_t* runs = nullptr;         // (first face, first vertex, end vertex) per run
     int n_runs = 0;
@@ -131,7 +132,7 @@ void fill_desc(QpsoSolveDev& h, const Mesh& m, const qpso_cluster* cl, const qps
     h.V_eff = (int32_t)m.v_prefix[h.F_eff - 1];
     h.faces = m.faces;
     h.corners = m.corners;
-    h.n_faces = (int32_t)m.F;
+    h.bounded = m.bounded ? 1 : 0;
     h.runs = m.runs;
     h.n_runs = m.n_runs;
     h.fx = p->cam.fx; h.fy = p->cam.fy; h.cx = p->cam.cx; h.cy = p->cam.cy;
@@ -629,6 +630,7 @@ int qpso_mesh_upload(qpso_ctx* ctx, const float* soa, uint32_t n_faces, uint32_t
     qpso_host::build_mesh_tables(soa, n_faces, verts, order, m.v_prefix, runs);
     m.n_runs = (int)(runs.size() / 3);
     m.V = (uint32_t)(verts.size() / 3);
+    m.bounded = qpso_host::bounded(verts);
     std::vector<float> corners;
     qpso_host::build_corner_table(soa, n_faces, order, corners);
     std::vector<QpsoFaceIdx> idx;

@@ -13,6 +13,7 @@
 #define QPSO_BEST_FIT_INIT 1.0e10f
 #define QPSO_FXP_LIMIT (1 << 30)  // degenerate guard on 28.4 coordinates
 #define QPSO_AREA_LIMIT (1 << 23) // degenerate guard on the union box area
+#define QPSO_MESH_BOUND 1e6f      // metres; a larger mesh takes the general projection
 
 // flags[] bits
 #define QPSO_FLAG_STALE_OVERFLOW 1
@@ -63,7 +64,7 @@ struct QpsoSolveDev {
     int32_t V_eff;   // unique vertices referenced by faces < F_eff (a prefix)
     const QpsoFaceIdx* faces;
     const float* corners;  // [F][3][4]: face f's corner j at corners[12 f + 4 j], (x, y, z, vertex index bits)
-    int32_t n_faces; // entries in `faces` (= F)
+    int32_t bounded; // every vertex coordinate is below QPSO_MESH_BOUND in magnitude
     // runs of consecutive faces whose corners lie in a short vertex range:
     // (first face, first vertex, end vertex) per run, for meshes whose
     // vertices do not fit the projected-vertex cache at once

@@ -494,7 +494,6 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     const Cam cam{S.fx, S.fy, S.cx, S.cy};
     const int Fe = S.F_eff;
     const QG QpsoFaceIdx* __restrict__ faces = (const QG QpsoFaceIdx*)S.faces;
-    const int n_faces = S.n_faces;
     const int32_t big_face = S.big_face;
 
     if (tid == 0) {
@@ -649,7 +648,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         }
         __syncthreads();
     };
-    const bool fast_ok = fast_inputs(pose, cam);
+    const bool fast_ok = S.bounded && fast_inputs(pose, cam);
     if (fast_ok) pass_a(std::false_type{});
     const bool fast = fast_ok && s_degen == 0;  // uniform
     if (!fast) {

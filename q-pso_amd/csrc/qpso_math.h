@@ -212,23 +212,26 @@ struct Cam {
     double fx, fy, cx, cy;
 };
 
-// A vertex in the camera's frame.  kBounded (fast_inputs): the rotation's
-// 2 (q x v) takes its factor into the constants, where doubling is exact; it is
-// not for a quaternion that overflows doubled.
+// A vertex in the camera's frame.  kBounded (fast_inputs): the factor of the
+// rotation's 2 (q x v) goes into the constants that multiply it.  Doubling a
+// float is exact unless it overflows, so q0 (2 t) and (2 q0) t are one product,
+// and every rounding falls on the same number as in the other form.  (The
+// constants inside q x v may not take it: there a product below 2^-126 rounds
+// differently doubled, and may turn a tie of the sum.)
 template <bool kBounded>
 QD void to_camera(const float pose[7], float vx, float vy, float vz, float& px, float& py, float& pz) {
     const float q0 = pose[3], q1 = pose[4], q2 = pose[5], q3 = pose[6];
-    const float a = kBounded ? 2.0f : 1.0f, b = kBounded ? 1.0f : 2.0f;
-    const float d1 = a * q1, d2 = a * q2, d3 = a * q3;
-    const float t0 = b * __builtin_fmaf(d2, vz, -(d3 * vy));
-    const float t1 = b * __builtin_fmaf(-d1, vz, d3 * vx);
-    const float t2 = b * __builtin_fmaf(d1, vy, -(d2 * vx));
-    const float k0 = __builtin_fmaf(q2, t2, -(q3 * t1));
-    const float k1 = __builtin_fmaf(-q1, t2, q3 * t0);
-    const float k2 = __builtin_fmaf(q1, t1, -(q2 * t0));
-    px = __builtin_fmaf(q0, t0, vx) + k0;
-    py = __builtin_fmaf(q0, t1, vy) + k1;
-    pz = __builtin_fmaf(q0, t2, vz) + k2;
+    const float a = kBounded ? 1.0f : 2.0f, b = kBounded ? 2.0f : 1.0f;
+    const float t0 = a * __builtin_fmaf(q2, vz, -(q3 * vy));
+    const float t1 = a * __builtin_fmaf(-q1, vz, q3 * vx);
+    const float t2 = a * __builtin_fmaf(q1, vy, -(q2 * vx));
+    const float e0 = b * q0, e1 = b * q1, e2 = b * q2, e3 = b * q3;
+    const float k0 = __builtin_fmaf(e2, t2, -(e3 * t1));
+    const float k1 = __builtin_fmaf(-e1, t2, e3 * t0);
+    const float k2 = __builtin_fmaf(e1, t1, -(e2 * t0));
+    px = __builtin_fmaf(e0, t0, vx) + k0;
+    py = __builtin_fmaf(e0, t1, vy) + k1;
+    pz = __builtin_fmaf(e0, t2, vz) + k2;
     px += pose[0];
     py += pose[1];
     pz += pose[2];
@@ -289,13 +292,15 @@ QD float max_nan(float a, float b) {
 QD uint32_t pack_fast(float x, float y) {
     return __builtin_amdgcn_perm(__float_as_uint(y + kRound), __float_as_uint(x + kRound), 0x05040100u);
 }
-// whether the pose and the camera are numbers that vertex_fast takes
+// Whether the pose and the camera are numbers that vertex_fast takes, for a
+// mesh within QPSO_MESH_BOUND: q x v stays below 2e21 in magnitude, and what it
+// is multiplied into below 1e37.
 QD bool fast_inputs(const float pose[7], const Cam& c) {
     const double m = __builtin_fabs(c.fx) + __builtin_fabs(c.fy) + __builtin_fabs(c.cx) + __builtin_fabs(c.cy);
     float p = 0.0f;
 #pragma unroll
     for (int d = 0; d < 7; ++d) p += __builtin_fabsf(pose[d]);
-    return m < 1e30 && p < 1e30f;
+    return m < 1e30 && p < 1e15f;
 }
 
 // Fixed-point face: 28.4 vertices and the integer bbox (main.h:1326-1353).

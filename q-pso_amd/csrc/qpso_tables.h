@@ -141,6 +141,13 @@ inline void build_mesh_tables(const float* A, uint32_t F, std::vector<float>& ve
     build_runs(tri, F, runs);
 }
 
+// Whether every coordinate is below QPSO_MESH_BOUND in magnitude (NaN is not).
+inline bool bounded(const std::vector<float>& verts) {
+    for (const float v : verts)
+        if (!(v > -QPSO_MESH_BOUND && v < QPSO_MESH_BOUND)) return false;
+    return true;
+}
+
 // The raster table as the device reads it: vertex indices modulo 65536.
 inline void build_index_table(const std::vector<QpsoFaceRef>& order, std::vector<QpsoFaceIdx>& out) {
     out.resize(order.size());
