@@ -349,11 +349,11 @@ __device__ __forceinline__ void step_in_launch(const QpsoSolveDev& S, int p, int
 
 // Waves per SIMD when as many workgroups as the LDS allows share a CU (160
 // KiB of LDS, 4 SIMDs): the register budget both bodies of a windowed
-// kernel must fit, so that its extra code never costs a workgroup.  Left
-// free (1) for 256-thread workgroups: the 10,112-word tile would need 4 waves
-// and 128 registers, which its bodies exceed without spilling at 3.
+// kernel must fit, so that its extra code never costs a workgroup.  One fewer
+// for 256-thread workgroups of the 10,112-word tile: at 4 waves and 128
+// registers their bodies would spill, at 3 they hardly do.
 constexpr int rf_waves_per_simd(int bt, int cap) {
-    return bt >= 512 ? (bt / 256) * ((160 * 1024) / (cap * 4 + 512)) : 1;
+    return bt >= 512 ? (bt / 256) * ((160 * 1024) / (cap * 4 + 512)) : cap <= 10112 ? 3 : 2;
 }
 
 typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
@@ -366,6 +366,12 @@ __device__ __forceinline__ uint32_t pack_xy(int32_t X, int32_t Y) {  // X | Y <<
 // keep: it starts above row b1; down: it ends below it (b1w = b1 << 16; the y
 // half decides a 32-bit comparison against it).  20 instructions instead of 48
 // on 32-bit coordinates.
+//   kWide: corners clamped to kHalf (2,047 pixels).  Clamped or not, a corner lies
+// on the same side of the region's edges, so only the way the face looks needs
+// more: the 32-bit products of face_front, or, with a clamped corner, the face
+// counts as front-facing and is told when it is drawn.
+constexpr int32_t kHalf = 32767 - 15;
+template <bool kWide>
 __device__ __forceinline__ bool cull_packed(uint32_t pa, uint32_t pb, uint32_t pc, uint32_t lo, uint32_t hi,
                                             int32_t b1w, bool& keep, bool& down) {
     const i16x2 A = __builtin_bit_cast(i16x2, pa), B = __builtin_bit_cast(i16x2, pb), C = __builtin_bit_cast(i16x2, pc);
@@ -375,12 +381,26 @@ __device__ __forceinline__ bool cull_packed(uint32_t pa, uint32_t pb, uint32_t p
     const i16x2 d = __builtin_elementwise_min(mx, __builtin_bit_cast(i16x2, hi)) -
                     __builtin_elementwise_max(mn, __builtin_bit_cast(i16x2, lo));
     const bool in = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(d, c1)) == 0x00010001u;
-    const int32_t ab = __builtin_bit_cast(int32_t, A - B), ca = __builtin_bit_cast(int32_t, C - A);
-    // DX12 DY31 > DX31 DY12: both products below 2^30
-    const bool front = __mul24((ab << 16) >> 16, ca >> 16) > __mul24((ca << 16) >> 16, ab >> 16);
+    bool front;
+    if (kWide) {
+        const auto x = [](uint32_t p) { return (int32_t)(p << 16) >> 16; };
+        const auto y = [](uint32_t p) { return (int32_t)p >> 16; };
+        front = wsub(wmul(x(pa) - x(pb), y(pc) - y(pa)), wmul(x(pc) - x(pa), y(pa) - y(pb))) > 0;
+        // clamped: a bound of 2,047 either way (bit 11 of it plus one)
+        const i16x2 far = __builtin_elementwise_max(mx, -mn) + c1;
+        front = front || (__builtin_bit_cast(uint32_t, far) & 0x08000800u) != 0u;
+    } else {
+        const int32_t ab = __builtin_bit_cast(int32_t, A - B), ca = __builtin_bit_cast(int32_t, C - A);
+        // DX12 DY31 > DX31 DY12: both products below 2^30
+        front = __mul24((ab << 16) >> 16, ca >> 16) > __mul24((ca << 16) >> 16, ab >> 16);
+    }
     keep = __builtin_bit_cast(int32_t, mn) < b1w;
     down = __builtin_bit_cast(int32_t, mx) > (b1w | 0xffff);
     return in && front;
+}
+__device__ __forceinline__ int32_t clamp_half(int32_t a) { return min(max(a, -kHalf), kHalf); }
+__device__ __forceinline__ float clamp_half(float a) {
+    return __builtin_amdgcn_fmed3f(a, -(float)kHalf, (float)kHalf);
 }
 __device__ __forceinline__ void todo_mask(uint64_t todo, bool reach, bool keep, bool down, uint64_t& m, uint64_t& lm) {
     const uint64_t r = todo & __ballot(reach);
@@ -413,8 +433,12 @@ struct RfLds {
 
 // WIN: the body that can draw a mesh window by window (larger than the vertex
 // cache); the other one keeps the cached path free of it.
-template <int BT, int CAP, int MODE>
-__device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves, const QpsoItem* __restrict__ items,
+// WIDE: the body for a particle drawn in windows without later bits whose box
+// leaves the packed cache's range; the ordinary one returns true for it, having written nothing
+// but the box, and is free of what it needs (in one body the ordinary cull ran
+// 3 % slower, 50k faces, 128 particles).
+template <int BT, int CAP, int MODE, bool WIDE>
+__device__ __forceinline__ bool rf_body(const QpsoSolveDev* __restrict__ solves, const QpsoItem* __restrict__ items,
                                         RfLds<CAP>& sh, int it) {
     constexpr bool WIN = MODE >= 1;     // meshes beyond the vertex cache, window by window
     constexpr bool FRAMES = MODE == 2;  // and the frame dump (stage calls)
@@ -481,14 +505,14 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             carried[j] = k < n_old ? load_stale(old, k) : QpsoStale{0, 0};
         }
     }
-    if (iter >= S.I) return;  // this solve has finished (batched runs)
+    if (iter >= S.I) return false;  // this solve has finished (batched runs)
     // each instantiation only for the meshes and outputs it handles
     if ((!WIN && Ve > kWin) || (!FRAMES && S.dbg_frames)) {
         if (tid == 0) {
             fit_out[p] = __builtin_nanf("");
             atomicOr(S.flags, QPSO_FLAG_LAUNCH);
         }
-        return;
+        return false;
     }
 
     const Cam cam{S.fx, S.fy, S.cx, S.cy};
@@ -519,7 +543,16 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     // second word holds Z (zc); otherwise a drawn face's corner depths are
     // projected again from the face's corner table.  A particle with vertices
     // beyond the halves, or a box too wide for their differences, projects
-    // every face from the corner table instead (pack = false).
+    // every face from the corner table instead (pack = false): once, since the
+    // later bits (below) name what the next bands draw.  A mesh in windows that
+    // has more faces than those bits hold clamps its coordinates to the
+    // halves (WIDE): whether a face reaches the band and the tile is still exact,
+    // and which way it looks is told from the corner table when it is drawn
+    // if a corner was clamped.  (Such boxes, 512 particles, a 300 px rect, a launch:
+    // 100k faces, 512 threads and 20,224 words, corner table 1,970 us, clamped
+    // 1,240; 256 threads and 10,112 words 4,910 and 1,960.  With the bits the
+    // LDS that no cache takes saves bands: 60k faces, 512 threads and 20,224
+    // words, corner table 1,030 us, clamped 1,110.)
     //   Any mesh is kept whole (cached) that leaves the rect a depth region of
     // half its size, or that is no larger than the packed window of kWin words
     // twice.  A larger one is cut on the host into runs of faces whose
@@ -590,13 +623,13 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             if (kGeneral) {
                 int32_t X, Y;
                 vertex_fixed(pose, x, y, z, cam, X, Y, Z);
-                xy = pack_xy(X, Y);
+                xy = WIDE ? pack_xy(clamp_half(X), clamp_half(Y)) : pack_xy(X, Y);
                 xl = min(xl, X); xh = max(xh, X);
                 yl = min(yl, Y); yh = max(yh, Y);
             } else {
                 float a, b;
                 ok = ok & vertex_fast(pose, x, y, z, cam16, a, b, Z);
-                xy = pack_fast(a, b);
+                xy = WIDE ? pack_fast(clamp_half(a), clamp_half(b)) : pack_fast(a, b);
                 // a coordinate that is no number (a quaternion or a mesh of
                 // 1e20 overflows in X and Y alone) fails the range test too
                 fxl = min_nan(fxl, a); fxh = max_nan(fxh, a);
@@ -680,14 +713,20 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             S.stale_cnt[par ^ 1][p] = 0;
             atomicAdd(&S.counters[2], 1ull);
         }
-        return;
+        return false;
     }
 
     // (X + 15) >> 4 >= -2047 gives X >= -32767 and <= 2046 gives X <= 32736:
     // every cached vertex fits the 16-bit halves; a box of at most 2046 pixels
     // a side keeps their differences and (a + 15) in 16 bits too
-    if (!(ax0 >= -2047 && ax1 <= 2046 && ay0 >= -2047 && ay1 <= 2046 && ax1 - ax0 <= 2046 && ay1 - ay0 <= 2046))
+    if (!WIDE &&
+        !(ax0 >= -2047 && ax1 <= 2046 && ay0 >= -2047 && ay1 <= 2046 && ax1 - ax0 <= 2046 && ay1 - ay0 <= 2046)) {
+        if (WIN && runs && l_words == 0) {
+            __syncthreads();  // every thread has read the box
+            return true;
+        }
         pack = false;
+    }
     const int32_t W = (int32_t)W64, H = (int32_t)H64;
     const int32_t A = W * H;
     const int32_t T = ((A + 1023) >> 10) << 10;  // NumIters * 1024 (main.cu:621-623)
@@ -798,10 +837,10 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     // coordinates, one 16-byte entry per corner, which carries the vertex
     // index: the face table entry is not read); or all three projected
     // again (in_cache false: the same arithmetic, so the same bits)
-    bool in_cache = pack;
+    bool in_cache = pack && !WIDE;
     auto draw_face = [&](int32_t f, Face& fc) {
         if (!in_cache) {
-            face_project(S.corners, f, pose, cam, fc);
+            face_project(S.corners, f, pose, cam, cam16, fast, fc);
             return;
         }
         if (zc) {
@@ -836,7 +875,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
     };
     // a queued face, drawn after its window
     auto queued_face = [&](int32_t f, Face& fc) {
-        if (WIN && runs) face_project(S.corners, f, pose, cam, fc);
+        if (WIN && runs) face_project(S.corners, f, pose, cam, cam16, fast, fc);
         else draw_face(f, fc);
     };
     // per-pixel depth over [x0, x1) x [y0, y1): edge values at (x0, y0), per
@@ -1081,6 +1120,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             Face fc;
             Setup su;
             draw_face(i, fc);
+            if (WIDE && !face_front(fc)) return;
             face_setup(fc, su);
             const int32_t x0 = max(fc.minx, tx0), x1 = min(fc.maxx, tx1);
             const int32_t y0 = max(fc.miny, b0), y1 = min(fc.maxy, b1);
@@ -1161,7 +1201,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
         // a later band draws the faces of the later bits; it tests them (and
         // updates the bits) where a band follows and the cache holds them
         const bool direct = !first && lbits && !(cached && more);
-        in_cache = pack && (cached || !direct);
+        in_cache = pack && !WIDE && (cached || !direct);
         // packed bounds of the band's part of the tile: x | y << 16
         const uint32_t lo2 = (uint32_t)tx0 | ((uint32_t)b0 << 16), hi2 = (uint32_t)tx1 | ((uint32_t)ty1 << 16);
         const int32_t b1w = (int32_t)((uint32_t)b1 << 16);
@@ -1208,6 +1248,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                             const int v = v0 + j * BT;
                             float a, b, Z;
                             vertex_fast(pose, x[j], y[j], z[j], cam16, a, b, Z);
+                            if (WIDE) { a = clamp_half(a); b = clamp_half(b); }
                             if (v < vhi) vP[v - vlo] = pack_fast(a, b);
                             const int n = min(v + kP * BT, vhi - 1);
                             x[j] = wx[n]; y[j] = wy[n]; z[j] = wz[n];
@@ -1218,6 +1259,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                         int32_t X, Y;
                         float Z;
                         vertex_fixed(pose, wx[v], wy[v], wz[v], cam, X, Y, Z);
+                        if (WIDE) { X = clamp_half(X); Y = clamp_half(Y); }
                         vP[v - vlo] = pack_xy(X, Y);
                     }
                 }
@@ -1280,7 +1322,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                 for (int g = 0; g < kGroup; ++g) {
                     const int i = base + g * 64 + lane;
                     bool keep, down;
-                    const bool reach = cull_packed(pv[g][0], pv[g][1], pv[g][2], lo2, hi2, b1w, keep, down);
+                    const bool reach = cull_packed<WIDE>(pv[g][0], pv[g][1], pv[g][2], lo2, hi2, b1w, keep, down);
                     const uint64_t in = __ballot((uint32_t)(i - f_lo) < (uint32_t)(f_hi - f_lo)) & __ballot(reach);
                     m[g] = in & __ballot(keep);
                     lm[g] = in & __ballot(down);
@@ -1300,11 +1342,11 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
                                 const uint32_t vb = WIN ? (uint32_t)vbase : 0u;
                                 const qv2 e = load_ref(faces, i);
                                 const uint32_t x = (uint32_t)e.x, y = (uint32_t)e.y;
-                                reach = cull_packed(vP[(x - vb) & 0xffffu], vP[((x >> 16) - vb) & 0xffffu],
-                                                    vP[(y - vb) & 0xffffu], lo2, hi2, b1w, keep, down);
+                                reach = cull_packed<WIDE>(vP[(x - vb) & 0xffffu], vP[((x >> 16) - vb) & 0xffffu],
+                                                          vP[(y - vb) & 0xffffu], lo2, hi2, b1w, keep, down);
                             } else {
                                 Face fc;
-                                face_project(S.corners, i, pose, cam, fc);
+                                face_project(S.corners, i, pose, cam, cam16, fast, fc);
                                 reach = max(fc.minx, tx0) < min(fc.maxx, tx1) && fc.miny < ty1 && fc.maxy > b0 && face_front(fc);
                                 keep = fc.miny < b1;
                                 down = fc.maxy > b1;
@@ -1692,6 +1734,7 @@ __device__ __forceinline__ void rf_body(const QpsoSolveDev* __restrict__ solves,
             atomicAdd(&S.counters[1], s_px[1]);
         }
     }
+    return false;
 }
 
 // One workgroup per (solve, particle).  A launch whose solves include a mesh
@@ -1706,14 +1749,12 @@ void k_render_fitness(const QpsoSolveDev* __restrict__ solves, const QpsoItem* _
     // spills the body's registers
     if (it > 0 && !(it & QPSO_STEP_APART) && __builtin_amdgcn_readfirstlane(threadIdx.x) < 64)
         step_in_launch(solves[0], (int)blockIdx.x, it, sh.s_pose);
-    if (MODE == 1) {
-        const QpsoItem item = items ? items[blockIdx.x] : QpsoItem{0, (int32_t)blockIdx.x};
-        if (solves[item.solve].V_eff <= CAP / 6) {
-            rf_body<BT, CAP, 0>(solves, items, sh, it);
-            return;
-        }
-    }
-    rf_body<BT, CAP, MODE>(solves, items, sh, it);
+    // (one path through both ordinary bodies to the wide one: with a return
+    // between them the compiler takes eleven registers more)
+    const QpsoItem item = items ? items[blockIdx.x] : QpsoItem{0, (int32_t)blockIdx.x};
+    const bool wide = MODE == 1 && solves[item.solve].V_eff <= CAP / 6 ? rf_body<BT, CAP, 0, false>(solves, items, sh, it)
+                                                                       : rf_body<BT, CAP, MODE, false>(solves, items, sh, it);
+    if (MODE >= 1 && __builtin_amdgcn_readfirstlane(wide)) rf_body<BT, CAP, MODE, MODE >= 1>(solves, items, sh, it);
 }
 
 // ------------------------------------------------------------------------
@@ -1835,7 +1876,7 @@ __global__ __launch_bounds__(BT) void k_render_fitness_wrap(const QpsoSolveDev* 
     unsigned long long px_r = 0;
     for (int f = tid; f < S.F_eff; f += BT) {
         Face fc;
-        face_project(S.corners, f, pose, cam, fc);
+        face_project(S.corners, f, pose, cam, Cam16{}, false, fc);
         if (!face_front(fc)) continue;
         Setup su;
         face_setup(fc, su);

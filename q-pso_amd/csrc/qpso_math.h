@@ -288,6 +288,8 @@ QD float max_nan(float a, float b) {
     asm("v_maximum3_f32 %0, %1, %2, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
+// such a coordinate rounded
+QD int32_t round_fast(float x) { return __float_as_int(x + kRound) - __float_as_int(kRound); }
 // X | Y << 16 of such coordinates
 QD uint32_t pack_fast(float x, float y) {
     return __builtin_amdgcn_perm(__float_as_uint(y + kRound), __float_as_uint(x + kRound), 0x05040100u);
@@ -333,18 +335,26 @@ QD int beyond_limit(int32_t xl, int32_t xh, int32_t yl, int32_t yh) {
 }
 
 // Face f projected from the corner table (corner j of face f at
-// corners[12 f + 4 j], (x, y, z, vertex index): one 16-byte load per corner).
-QD void face_project(const float* __restrict__ corners, int f, const float pose[7], const Cam& c, Face& fc) {
+// corners[12 f + 4 j], (x, y, z, vertex index): one 16-byte load per corner),
+// with the fast projection where all of the particle's vertices take it.
+QD void face_project(const float* __restrict__ corners, int f, const float pose[7], const Cam& c, const Cam16& c16,
+                     bool fast, Face& fc) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     const f4* __restrict__ cr = reinterpret_cast<const f4*>(corners) + 3 * (size_t)f;
+    f4 w[3];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const f4 w = cr[j];
-        float u, v, Z;
-        project(pose, w.x, w.y, w.z, c, u, v, Z);
-        fc.X[j] = rint_sat(16.0f * u);
-        fc.Y[j] = rint_sat(16.0f * v);
-        fc.Z[j] = Z;
+    for (int j = 0; j < 3; ++j) w[j] = cr[j];
+    if (fast) {  // uniform
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            float x, y;
+            vertex_fast(pose, w[j].x, w[j].y, w[j].z, c16, x, y, fc.Z[j]);
+            fc.X[j] = round_fast(x);
+            fc.Y[j] = round_fast(y);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) vertex_fixed(pose, w[j].x, w[j].y, w[j].z, c, fc.X[j], fc.Y[j], fc.Z[j]);
     }
     face_bbox(fc);
 }
