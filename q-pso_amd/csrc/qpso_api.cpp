@@ -408,14 +408,14 @@ int read_results(qpso_ctx* ctx, int n, qpso_solve* const* solves, qpso_result* o
     const hipStream_t st = ctx->stream;
     constexpr size_t kWords = 1024;  // a solve's part of the staging
     char* h = stage_for(ctx, kWords * n);
-    if (!h) return QPSO_E_NOMEM;
-    for (int i = 0; i < n; ++i) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; h && i < n && e == hipSuccess; ++i) {
         const ArenaLayout& L = solves[i]->L;
-        if (hipMemcpyAsync(h + kWords * i, solves[i]->arena + L.gbest, L.counters + 24 - L.gbest, hipMemcpyDeviceToHost,
-                           st) != hipSuccess)
-            return QPSO_E_HIP;
+        e = hipMemcpyAsync(h + kWords * i, solves[i]->arena + L.gbest, L.counters + 24 - L.gbest, hipMemcpyDeviceToHost, st);
     }
-    if (hipStreamSynchronize(st) != hipSuccess) return QPSO_E_HIP;
+    const hipError_t e2 = hipStreamSynchronize(st);  // whatever was queued has ended
+    if (!h) return QPSO_E_NOMEM;
+    if (e != hipSuccess || e2 != hipSuccess) return QPSO_E_HIP;
     int rc = QPSO_OK;
     for (int i = 0; i < n; ++i) {
         const ArenaLayout& L = solves[i]->L;
