@@ -279,8 +279,10 @@ hipError_t copy_on(hipStream_t st, void* dst, const void* src, size_t bytes, hip
     return e == hipSuccess ? hipStreamSynchronize(st) : e;
 }
 
-// Pinned staging of at least this many bytes (null if there is none to be had).
-char* stage_for(qpso_ctx* ctx, size_t bytes) {
+// Staging of at least this many bytes: the context's pinned memory, or, where
+// there is none to be had, `spare` (a pageable copy takes longer and works).
+// Either lasts until the call's copies have ended.
+char* stage_for(qpso_ctx* ctx, size_t bytes, std::vector<char>& spare) {
     if (bytes <= ctx->stage_bytes) return ctx->stage;
     if (ctx->stage) hipHostFree(ctx->stage);
     ctx->stage = nullptr;
@@ -289,7 +291,8 @@ char* stage_for(qpso_ctx* ctx, size_t bytes) {
     if (hipHostMalloc(reinterpret_cast<void**>(&ctx->stage), n) != hipSuccess) {
         hipGetLastError();
         ctx->stage = nullptr;
-        return nullptr;
+        spare.resize(bytes);
+        return spare.data();
     }
     ctx->stage_bytes = n;
     return ctx->stage;
@@ -407,14 +410,14 @@ int result_from(const ResultWords& w, qpso_result* out) {
 int read_results(qpso_ctx* ctx, int n, qpso_solve* const* solves, qpso_result* out) {
     const hipStream_t st = ctx->stream;
     constexpr size_t kWords = 1024;  // a solve's part of the staging
-    char* h = stage_for(ctx, kWords * n);
+    std::vector<char> spare;
+    char* const h = stage_for(ctx, kWords * n, spare);
     hipError_t e = hipSuccess;
-    for (int i = 0; h && i < n && e == hipSuccess; ++i) {
+    for (int i = 0; i < n && e == hipSuccess; ++i) {
         const ArenaLayout& L = solves[i]->L;
         e = hipMemcpyAsync(h + kWords * i, solves[i]->arena + L.gbest, L.counters + 24 - L.gbest, hipMemcpyDeviceToHost, st);
     }
     const hipError_t e2 = hipStreamSynchronize(st);  // whatever was queued has ended
-    if (!h) return QPSO_E_NOMEM;
     if (e != hipSuccess || e2 != hipSuccess) return QPSO_E_HIP;
     int rc = QPSO_OK;
     for (int i = 0; i < n; ++i) {
@@ -721,15 +724,12 @@ int create_solve(qpso_ctx* ctx, uint32_t mesh_id, const qpso_cluster* cl, const 
     int rc = QPSO_OK;
     // the descriptor, the crop and its rows open the arena: one copy
     const size_t up = s->L.obs_rows + rows.size() * 2;
-    if (char* h = stage_for(ctx, up)) {
-        std::memcpy(h + s->L.desc, &s->h, sizeof(QpsoSolveDev));
-        std::memcpy(h + s->L.obs, crop.data(), crop.size() * 2);
-        std::memcpy(h + s->L.obs_rows, rows.data(), rows.size() * 2);
-        if (copy_on(st, A, h, up, hipMemcpyHostToDevice) != hipSuccess)
-            rc = set_err(ctx, QPSO_E_HIP, "solve upload failed");
-    } else {
-        rc = set_err(ctx, QPSO_E_NOMEM, "no pinned memory for the upload");
-    }
+    std::vector<char> spare;
+    char* const h = stage_for(ctx, up, spare);
+    std::memcpy(h + s->L.desc, &s->h, sizeof(QpsoSolveDev));
+    std::memcpy(h + s->L.obs, crop.data(), crop.size() * 2);
+    std::memcpy(h + s->L.obs_rows, rows.data(), rows.size() * 2);
+    if (copy_on(st, A, h, up, hipMemcpyHostToDevice) != hipSuccess) rc = set_err(ctx, QPSO_E_HIP, "solve upload failed");
     if (rc) {
         free_arena(ctx, s->arena, st);
         hipStreamSynchronize(st);
@@ -1040,8 +1040,8 @@ int qpso_solve_eval_poses(qpso_solve* s, int n, const float* poses, float* fit, 
         ctx->work_bytes = bytes;
     }
     char* const W = ctx->work;
-    char* const h = stage_for(ctx, total);
-    if (!h) return set_err(ctx, QPSO_E_NOMEM, "no pinned memory for the poses");
+    std::vector<char> spare;
+    char* const h = stage_for(ctx, total, spare);
     int32_t* d_frames = nullptr;
     QpsoSolveDev tmp = s->h;
     tmp.fit = reinterpret_cast<float*>(W + o_fit);

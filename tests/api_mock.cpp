@@ -300,12 +300,39 @@ bool results_wait_on_failure() {
     return true;
 }
 
+// Without pinned memory every call works as with it.
+bool no_pinned_memory() {
+    g.no_pinned = true;
+    bool ok = false;
+    {
+        World w;
+        ok = [&] {
+            qpso_solve* s[2];
+            for (int i = 0; i < 2; ++i) {
+                const qpso_cluster c = w.cluster(200 + i, 300);
+                CHECK(qpso_solve_create(w.ctx, w.mesh, &c, &w.p, 0, &s[i]) == QPSO_OK);
+            }
+            qpso_result r[2];
+            CHECK(qpso_solve_run(s[0], r) == QPSO_OK && w.right(r[0], 200, 300));
+            CHECK(qpso_solve_run_batch(w.ctx, 2, s, r) == QPSO_OK && w.right(r[1], 201, 300));
+            CHECK(w.scores_right(s[1], 8));
+            const qpso_cluster c = w.cluster(50, 40);
+            CHECK(qpso_estimate_pose(w.ctx, w.mesh, &c, &w.p, r) == QPSO_OK && w.right(r[0], 50, 40));
+            for (auto* x : s) qpso_solve_destroy(x);
+            return true;
+        }();
+    }
+    g.no_pinned = false;
+    return ok;
+}
+
 struct Scenario {
     const char* name;
     bool (*run)();
 };
 const Scenario kScenarios[] = {
     {"results_wait_on_failure", results_wait_on_failure},
+    {"no_pinned_memory", no_pinned_memory},
 };
 
 }  // namespace
