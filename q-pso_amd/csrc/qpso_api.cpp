@@ -38,6 +38,9 @@ constexpr int kFrame = kRows * kCols;
 constexpr int kStaleCap = QPSO_STALE_CAP;
 constexpr int kMaxIters = 1 << 20;          // iterations per solve
 constexpr size_t kMaxRand = size_t(1) << 30;  // random-table entries (4 GiB)
+// a context's pinned staging: 65,535 poses with their boxes and fitness, a
+// frame's crop with its prefix counts (1.3 MB), the results of 3,072 solves
+constexpr size_t kStageBytes = size_t(3) << 20;
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
@@ -215,12 +218,13 @@ struct qpso_ctx {
     // Host copies of the calls on `stream`: a call's inputs go up and its
     // results come down as one copy each through pinned memory (a pageable
     // copy takes several times a pinned one's time, and a solve had three
-    // each way).  `work`: poses in, boxes and fitness out of
-    // qpso_solve_eval_poses.  Both are used under `mu` by calls that end
-    // synchronised, grow to the largest call (at most a frame's crop, 65,535
-    // particles' poses) and go with the context.
+    // each way).  It has one size (kStageBytes) from the context's start:
+    // growing it frees pinned memory, which waits for the whole device, and
+    // the serving thread creates solves.  `work`: poses in, boxes and fitness
+    // out of qpso_solve_eval_poses, from the arenas' pool; it grows to the
+    // largest call (at most 65,535 particles' poses).  Both are used under `mu`
+    // by calls that end synchronised and go with the context.
     char* stage = nullptr;
-    size_t stage_bytes = 0;
     char* work = nullptr;
     size_t work_bytes = 0;
 };
@@ -279,23 +283,13 @@ hipError_t copy_on(hipStream_t st, void* dst, const void* src, size_t bytes, hip
     return e == hipSuccess ? hipStreamSynchronize(st) : e;
 }
 
-// Staging of at least this many bytes: the context's pinned memory, or, where
-// there is none to be had, `spare` (a pageable copy takes longer and works).
-// Either lasts until the call's copies have ended.
+// Staging of this many bytes: the context's pinned memory, or `spare` where that
+// is too small or there is none (a pageable copy takes longer and works).  Either
+// lasts until the call's copies have ended.
 char* stage_for(qpso_ctx* ctx, size_t bytes, std::vector<char>& spare) {
-    if (bytes <= ctx->stage_bytes) return ctx->stage;
-    if (ctx->stage) hipHostFree(ctx->stage);
-    ctx->stage = nullptr;
-    ctx->stage_bytes = 0;
-    const size_t n = align_up(std::max(bytes, size_t(64) << 10), size_t(64) << 10);
-    if (hipHostMalloc(reinterpret_cast<void**>(&ctx->stage), n) != hipSuccess) {
-        hipGetLastError();
-        ctx->stage = nullptr;
-        spare.resize(bytes);
-        return spare.data();
-    }
-    ctx->stage_bytes = n;
-    return ctx->stage;
+    if (ctx->stage && bytes <= kStageBytes) return ctx->stage;
+    spare.resize(bytes);
+    return spare.data();
 }
 
 // A solve arena: from the context's pool in the order of its stream (the
@@ -589,6 +583,10 @@ int qpso_create(int device, qpso_ctx** out) {
             hipGetLastError();  // without a pool the arenas come from hipMalloc
         }
     }
+    if (hipHostMalloc(reinterpret_cast<void**>(&ctx->stage), kStageBytes) != hipSuccess) {
+        hipGetLastError();
+        ctx->stage = nullptr;
+    }
     // with this device current: its copy of the no-allocation scratch
     void* scratch = nullptr;
     if (qpso_launch::scratch_address(device, &scratch) == hipSuccess) ctx->scratch = static_cast<char*>(scratch);
@@ -609,7 +607,7 @@ int qpso_destroy(qpso_ctx* ctx) {
     for (auto& kv : ctx->meshes) free_mesh(kv.second);
     for (auto& kv : ctx->rand_cache) hipFree(kv.second.d);
     if (ctx->stage) hipHostFree(ctx->stage);
-    if (ctx->work) hipFree(ctx->work);
+    if (ctx->work) free_arena(ctx, ctx->work, ctx->stream);
     if (ctx->pool) {
         hipDeviceSynchronize();
         hipMemPoolDestroy(ctx->pool);
@@ -1029,11 +1027,11 @@ int qpso_solve_eval_poses(qpso_solve* s, int n, const float* poses, float* fit, 
     const size_t o_fit = align_up(up, 256), o_box = align_up(o_fit + sizeof(float) * (size_t)n, 16);
     const size_t total = o_box + sizeof(int32_t) * 4 * (size_t)n;
     if (total > ctx->work_bytes) {
-        if (ctx->work) hipFree(ctx->work);
+        if (ctx->work) free_arena(ctx, ctx->work, st);
         ctx->work = nullptr;
         ctx->work_bytes = 0;
         const size_t bytes = align_up(total, size_t(64) << 10);
-        if (hipMalloc(reinterpret_cast<void**>(&ctx->work), bytes) != hipSuccess) {
+        if (alloc_arena(ctx, bytes, &ctx->work) != hipSuccess) {
             ctx->work = nullptr;
             return set_err(ctx, QPSO_E_NOMEM, "pose evaluation workspace");
         }
@@ -1246,7 +1244,8 @@ namespace {
 // steps are enqueued without a round trip.  A solve's last step is followed
 // on its lane by the copies of its result words into pinned host memory and
 // an event; its arena goes back to the context's pool in the lane's order.
-// Nothing in the loop waits for the device except a failure path.
+// Nothing in the loop waits for the device except a failure path, work tables
+// that have to grow, and the release of a random table beyond the idle ones kept.
 struct HipDev {
     using Solve = qpso_solve;
     struct Job {

@@ -326,6 +326,48 @@ bool no_pinned_memory() {
     return ok;
 }
 
+// Pinned memory is taken once, with the context: no call waits for the device
+// to grow it (the serving thread creates solves of any crop), and neither do
+// larger scorings.
+bool staging_keeps_its_size() {
+    World w;
+    w.p.n_iters = 1;
+    int mallocs = 0, host_frees = 0, frees = 0;
+    for (int k = 1; k <= 8; ++k) {
+        const int cw = 80 * k, ch = 60 * k;
+        const qpso_cluster c = w.cluster(cw, ch);
+        qpso_solve* s = nullptr;
+        w.p.n_particles = k == 8 ? 65535 : 1000 * k;
+        CHECK(qpso_solve_create(w.ctx, w.mesh, &c, &w.p, 0, &s) == QPSO_OK);
+        qpso_result r{};
+        CHECK(qpso_solve_run(s, &r) == QPSO_OK && w.right(r, cw, ch));
+        CHECK(w.scores_right(s, w.p.n_particles));
+        CHECK(w.scores_right(s, 3));
+        qpso_solve_destroy(s);
+        if (k == 1) {
+            mallocs = g.host_mallocs;
+            host_frees = g.host_frees;
+            frees = g.frees;
+        }
+        CHECK(g.host_mallocs == mallocs && g.host_frees == host_frees && g.frees == frees);
+    }
+    return true;
+}
+
+// More results than the staging holds.
+bool many_results() {
+    World w;
+    constexpr int kN = 3500;
+    const qpso_cluster c = w.cluster(9, 5);
+    std::vector<qpso_solve*> s(kN);
+    for (auto& x : s) CHECK(qpso_solve_create(w.ctx, w.mesh, &c, &w.p, 0, &x) == QPSO_OK);
+    std::vector<qpso_result> r(kN);
+    CHECK(qpso_solve_run_batch(w.ctx, kN, s.data(), r.data()) == QPSO_OK);
+    for (auto& x : r) CHECK(w.right(x, 9, 5));
+    for (auto* x : s) qpso_solve_destroy(x);
+    return true;
+}
+
 struct Scenario {
     const char* name;
     bool (*run)();
@@ -333,6 +375,8 @@ struct Scenario {
 const Scenario kScenarios[] = {
     {"results_wait_on_failure", results_wait_on_failure},
     {"no_pinned_memory", no_pinned_memory},
+    {"staging_keeps_its_size", staging_keeps_its_size},
+    {"many_results", many_results},
 };
 
 }  // namespace
