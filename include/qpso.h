@@ -276,9 +276,11 @@ int qpso_server_stats_get(qpso_server* sv, qpso_server_stats* st);
  * on the server may start once destroy has begun. */
 int qpso_server_destroy(qpso_server* sv);
 
-/* Device bytes of one solve's own arena (observed crop, swarm state, carried
- * pixels), the admission unit; its random table is shared and counted
- * separately (see qpso_server_create). */
+/* Device bytes of a served solve's own arena (observed crop, swarm state,
+ * carried pixels), the admission unit; its random table is shared and counted
+ * separately (see qpso_server_create).  A solve of qpso_solve_create also holds
+ * its traces, if it has them, and, with offframe = 0 and up to 4,096 particles,
+ * second buffers of pos, fit and gbest: 32 bytes a particle and at most 1 KiB. */
 uint64_t qpso_solve_bytes(const qpso_params* p, const int32_t rect[4]);
 
 #ifdef __cplusplus

@@ -368,6 +368,30 @@ bool many_results() {
     return true;
 }
 
+// qpso_solve_bytes is a served solve's arena; one of up to 4,096 particles that
+// may run on its own takes 32 bytes a particle and at most 1 KiB more.
+bool arena_bytes() {
+    World w;
+    const qpso_cluster c = w.cluster(33, 21);
+    for (const int n : {1, 8, 65, 257, 4096, 4097}) {
+        w.p.n_particles = n;
+        const uint64_t bytes = qpso_solve_bytes(&w.p, c.rect);
+        qpso_solve* s = nullptr;
+        CHECK(qpso_solve_create(w.ctx, w.mesh, &c, &w.p, 0, &s) == QPSO_OK);
+        CHECK(g.last_arena >= bytes + (n <= 4096 ? 32 * n : 0) && g.last_arena <= bytes + (n <= 4096 ? 32 * n + 1024 : 0));
+        qpso_solve_destroy(s);
+        qpso_server* sv = nullptr;
+        CHECK(qpso_server_create(w.ctx, uint64_t(1) << 32, &sv) == QPSO_OK);
+        uint64_t t = 0;
+        qpso_result r{};
+        CHECK(qpso_server_submit(sv, w.mesh, &c, &w.p, &t) == QPSO_OK);
+        CHECK(qpso_server_wait(sv, t, &r) == QPSO_OK && w.right(r, 33, 21));
+        qpso_server_destroy(sv);
+        CHECK(g.last_arena == bytes);
+    }
+    return true;
+}
+
 struct Scenario {
     const char* name;
     bool (*run)();
@@ -377,6 +401,7 @@ const Scenario kScenarios[] = {
     {"no_pinned_memory", no_pinned_memory},
     {"staging_keeps_its_size", staging_keeps_its_size},
     {"many_results", many_results},
+    {"arena_bytes", arena_bytes},
 };
 
 }  // namespace

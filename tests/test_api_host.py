@@ -15,7 +15,8 @@ INC = ["-I", os.path.join(ROCM, "include"), "-I", os.path.join(REPO, "include"),
 FLAGS = ["-std=c++17", "-O1", "-g", "-ffp-contract=off", "-fwrapv", "-Wno-unused-result", "-D__HIP_PLATFORM_AMD__", "-fno-omit-frame-pointer",
          "-fsanitize=address,undefined", "-fno-sanitize-recover=all"]
 
-SCENARIOS = ["results_wait_on_failure", "no_pinned_memory", "staging_keeps_its_size", "many_results"]
+SCENARIOS = ["results_wait_on_failure", "no_pinned_memory", "staging_keeps_its_size", "many_results",
+             "arena_bytes"]
 
 
 @pytest.fixture(scope="module")
