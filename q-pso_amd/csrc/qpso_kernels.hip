@@ -791,6 +791,15 @@ __device__ __forceinline__ bool rf_body(const QpsoSolveDev* __restrict__ solves,
     int32_t v_words = !pack ? 0 : zc ? 2 * VC : VC;
     bool lbits = region + TW + 8 > CAP - kFixed - (win ? kMinVC : v_words);
     lbits = lbits && l_words > 0;
+    // Four waves hardly hide what drawing from the corner table waits for: with a
+    // cache they cull every band from it, unless less than half of the box
+    // lies in the tile.  (A 300 px rect, 30k faces, 512 particles, a launch by the
+    // bits and from the cache: 256 threads and 10,112 words 1,320 and 920 us, and
+    // 20,224 words 630 and 520, 512 threads 465 and 433, 1,024 threads 305 and
+    // 332; 100k faces, 2,048 particles, 200 iterations on 1,024 threads 362 and
+    // 396 ms.  An object half off the frame, 12k faces, 256 threads and 10,112
+    // words: 330 and 410 us.)
+    if (BT <= 256 && pack && 2 * TW * TH >= (ax1 - ax0) * (ay1 - ay0)) lbits = false;
     if (win) {
         // the largest window, up to 2 kWin, that costs no band: projecting
         // and culling a band's windows again costs more than shorter windows
