@@ -493,7 +493,8 @@ int launch_solve(qpso_solve* s, hipStream_t st) {
 }
 
 // The plain run as one graph launch (captured at the first run, and again
-// after the configuration changes): 2I + 1 kernels without host launch cost.
+// after the configuration changes), its kernels without host launch cost: I + 2
+// with the PSO step inside the render launches, 2I + 1 without.
 int run_solve_graph(qpso_solve* s, hipStream_t st) {
     qpso_ctx* ctx = s->ctx;
     if (!s->exec) {

@@ -37,7 +37,6 @@ constexpr int kCols = 640;
 // Global-memory pointers: loads through them cannot alias LDS, so the compiler
 // may move them across LDS stores and atomics (generic pointers could).
 #define QG __attribute__((address_space(1)))
-typedef int32_t qv4 __attribute__((ext_vector_type(4)));
 typedef int32_t qv2 __attribute__((ext_vector_type(2)));
 // a face's three vertex indices modulo 65536: x = v0 | v1 << 16, y = v2
 __device__ __forceinline__ qv2 load_ref(const QG QpsoFaceIdx* p, int i) { return reinterpret_cast<const QG qv2*>(p)[i]; }
@@ -263,8 +262,7 @@ __device__ __forceinline__ void step_particle(const QpsoSolveDev& S, Particle& q
         }
     } else {
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
-        rotation_to(k == 0 ? &B[3] : &gb[3], &P[3], k == 0 ? wc : ws);
+        for (int k = 0; k < 2; ++k) rotation_to(k == 0 ? &B[3] : &gb[3], &P[3], k == 0 ? wc : ws);
     }
     V[3] = 0.0f;
 #pragma unroll
@@ -416,7 +414,8 @@ __device__ __forceinline__ uint64_t uniform64(uint64_t v) {  // a wave-uniform v
 // it may run.
 template <int CAP>
 struct RfLds {
-    __attribute__((aligned(16))) int32_t lds[CAP];  // [vertex cache: (X, Y) pairs, Z] [depth tile]
+    // [vertex cache: X | Y << 16, and Z with room] [queues] [rings] [later bits] [depth tile]
+    __attribute__((aligned(16))) int32_t lds[CAP];
     int32_t s_box[4];    // rendered AABB: minX, maxX, minY, maxY
     int32_t s_stale[4];  // carried pixels inside the union box: x0, x1, y0, y1 (inclusive)
     int32_t s_degen;
@@ -609,7 +608,7 @@ __device__ __forceinline__ bool rf_body(const QpsoSolveDev* __restrict__ solves,
     //      the pass runs again with the general one.  The pass is issue-bound:
     //      28.4k -> 25.4k clocks a workgroup for 50k faces, 55k -> 43k for
     //      100k; a solve of 256 particles and 10k faces 8.13 -> 7.90 ms.
-    const Cam16 cam16{16.0 * cam.fx, 16.0 * cam.fy, 16.0 * cam.cx, 16.0 * cam.cy};
+    const Cam cam16{16.0 * cam.fx, 16.0 * cam.fy, 16.0 * cam.cx, 16.0 * cam.cy};
     auto pass_a = [&](auto general) {
         constexpr bool kGeneral = decltype(general)::value;
         // faces [0, Fe) use exactly the vertices [0, Ve); their bbox extremes
@@ -1050,8 +1049,8 @@ __device__ __forceinline__ bool rf_body(const QpsoSolveDev* __restrict__ solves,
     // reaches rows below the band, set while a band culls; the next band
     // takes only those faces.  With windows a later band draws them straight
     // from the corner table (no window is projected or culled again); without
-    // the bits (more faces than kLater words hold) it culls every window again
-    // but those none of whose faces reached later rows (bit w of wmask; wslot:
+    // the bits (lbits above) it culls every face again, of windows but
+    // those none of whose faces reached later rows (bit w of wmask; wslot:
     // the windows drawn so far mod 3, the slot of s_later the current one
     // uses).
     uint64_t wmask = ~0ull;
@@ -1885,7 +1884,7 @@ __global__ __launch_bounds__(BT) void k_render_fitness_wrap(const QpsoSolveDev* 
     unsigned long long px_r = 0;
     for (int f = tid; f < S.F_eff; f += BT) {
         Face fc;
-        face_project(S.corners, f, pose, cam, Cam16{}, false, fc);
+        face_project(S.corners, f, pose, cam, cam, false, fc);
         if (!face_front(fc)) continue;
         Setup su;
         face_setup(fc, su);

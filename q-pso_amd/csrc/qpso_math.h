@@ -251,33 +251,25 @@ QD void project(const float pose[7], float vx, float vy, float vz, const Cam& c,
 // (the factor 16 taken into the camera, exact), valid where ok returns true
 // and both stay below kFastLimit in magnitude.  There adding kRound rounds
 // them half to even into the low mantissa bits, the 16-bit half directly.
-struct Cam16 {
-    double fx, fy, cx, cy;
-};
 constexpr float kFastLimit = 0x1p22f;
 constexpr float kRound = 0x1.8p23f;
-QD bool vertex_fast(const float pose[7], float vx, float vy, float vz, const Cam16& c, float& x, float& y, float& Z) {
+QD bool vertex_fast(const float pose[7], float vx, float vy, float vz, const Cam& c16, float& x, float& y, float& Z) {
     float px, py, pz, e;
     to_camera<true>(pose, vx, vy, vz, px, py, pz);
     const float r = rcp_newton(pz, e);
-    x = (float)__builtin_fma(c.fx, (double)(px * r), c.cx);
-    y = (float)__builtin_fma(c.fy, (double)(py * r), c.cy);
+    x = (float)__builtin_fma(c16.fx, (double)(px * r), c16.cx);
+    y = (float)__builtin_fma(c16.fy, (double)(py * r), c16.cy);
     Z = 1000.0f * pz;
     return __builtin_fabsf(e) < kRcpOk;
 }
-// minimum and maximum of numbers, one instruction (the library's forms first
-// quiet their operands; a NaN operand is passed over here too)
+// minimum of numbers, one instruction (the library's form first quiets its
+// operands; a NaN operand is passed over here too)
 QD float min_num(float a, float b) {
     float r;
     asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
-QD float max_num(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-// and the forms that hand a NaN operand on, at the same rate
+// minimum and maximum that hand a NaN operand on, at the same rate
 QD float min_nan(float a, float b) {
     float r;
     asm("v_minimum3_f32 %0, %1, %2, %2" : "=v"(r) : "v"(a), "v"(b));
@@ -337,7 +329,7 @@ QD int beyond_limit(int32_t xl, int32_t xh, int32_t yl, int32_t yh) {
 // Face f projected from the corner table (corner j of face f at
 // corners[12 f + 4 j], (x, y, z, vertex index): one 16-byte load per corner),
 // with the fast projection where all of the particle's vertices take it.
-QD void face_project(const float* __restrict__ corners, int f, const float pose[7], const Cam& c, const Cam16& c16,
+QD void face_project(const float* __restrict__ corners, int f, const float pose[7], const Cam& c, const Cam& c16,
                      bool fast, Face& fc) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     const f4* __restrict__ cr = reinterpret_cast<const f4*>(corners) + 3 * (size_t)f;
